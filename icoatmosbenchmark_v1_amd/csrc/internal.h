@@ -193,6 +193,18 @@ __device__ __forceinline__ long xcd_contiguous(long b, long n)
     return (per > 0 && b < per * nxcd) ? (b % nxcd) * per + b / nxcd : b;
 }
 
+// As xcd_contiguous, in windows: `unit` consecutive logical work-groups share
+// an XCD, and the eight XCDs work on neighbouring units at the same time, so
+// that what a unit shares comes from one L2 while the chip as a whole sweeps
+// memory in order (eight distant ranges at once cost DRAM efficiency).  The
+// last n % (8 * unit) work-groups keep their index.
+__device__ __forceinline__ long xcd_windowed(long b, long n, long unit)
+{
+    constexpr long nxcd = 8;
+    const long win = nxcd * unit, w = b / win, r = b - w * win;
+    return b < n / win * win ? w * win + (r % nxcd) * unit + r / nxcd : b;
+}
+
 // Stores of outputs that no work-item of the same launch reads back carry the
 // nontemporal hint, so output streams of hundreds of MB do not evict the halo
 // rows and metrics that neighbouring work-groups re-read from L2.  Measured at

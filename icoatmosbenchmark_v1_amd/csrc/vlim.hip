@@ -13,19 +13,19 @@
 // last work-items.
 //
 // Many tracers (q(gall,kall,lall,ntr), NICAM's tracer-last layout) share ck
-// and d.  The batched kernel gives a work-item up to TB tracers of one
-// column run: per level it loads ck and d once and forms the
-// tracer-independent flags, Courant sums and zerosw once, then limits each
-// tracer with the single-tracer arithmetic.
+// and d: a work-group limits one tracer, and the tracers of one column block
+// and run are consecutive work-groups on one XCD, whose L2 serves ck and d to
+// all but the first.
+#include <type_traits>
+
 #include "internal.h"
 
 namespace nicam {
 namespace {
 
 constexpr int BLOCK = 256;
-#ifndef NICAM_VLIM_KC
-#define NICAM_VLIM_KC 4  // levels per run of the single-tracer kernel (0: runtime-length runs of 4); gl7: 4 164 us, 8 168, 16 168, runtime-length 169 (FP64)
-#endif
+constexpr int RUN_KC = 4;  // levels per run; gl7: 4 164 us, 8 168, 16 168, runtime-length 169 (FP64)
+constexpr int WIN = 4;     // column blocks an XCD takes at a time (gl7: 1 541 us for the vertical half, 4 530, 8 540)
 
 template <class T>
 __device__ __forceinline__ T dmin(T a, T b) { return (b < a) ? b : a; }
@@ -45,7 +45,7 @@ struct VlimArgs {
     int gall, kall, lall, gall_pl, have_pl;
     int kc, nrun;  // levels per work-item, runs per column
     T eps, big;
-    int ntr;          // tracers (batched kernel)
+    int ntr;          // tracers
     long ts, tps;     // tracer strides of the regular and pole fields
     uint32_t *mask, *mask_pl;  // clip bits (masked variant only; kc = 32)
 };
@@ -177,112 +177,55 @@ __device__ __forceinline__ void vlim_run_kc(T *__restrict__ q_h, const T *__rest
     }
 }
 
-// vlim_run for up to TB tracers (nb of them) of one column run; tracer b's
-// fields start b*ts elements after q / q_h.
-template <bool POLE, int TB, class T>
-__device__ __forceinline__ void vlim_run_multi(T *__restrict__ q_h, const T *__restrict__ q,
-                                               const T *__restrict__ d, const T *__restrict__ ck, size_t base,
-                                               size_t s, size_t ck2, int kb, int ke, T EPS, T BIG, int nb, long ts)
-{
-    int k = kb - 1;
-    T qkm1[TB], qk[TB], Qmin_km1[TB], Qmax_km1[TB];
-#pragma unroll
-    for (int b = 0; b < TB; ++b) {
-        const int bb = b < nb ? b : 0;  // idle slots repeat tracer 0 and store nothing
-        qkm1[b] = q[bb * ts + base + (size_t)(k - 1) * s];
-        qk[b] = q[bb * ts + base + (size_t)k * s];
-        Qmin_km1[b] = T(0);
-        Qmax_km1[b] = T(0);
-    }
-    T ck1k = ck[base + (size_t)k * s];
-    for (; k < ke; ++k) {
-        const size_t o = base + (size_t)k * s;
-        const T ck1kp1 = ck[o + s];
-        const T ck2k = ck[ck2 + o];
-        const T dk = d[o];
-        const T inflagL = T(0.5) - sign_half(ck1k);
-        const T inflagU = T(0.5) + sign_half(ck1kp1);
-        const T Cin = (inflagL)*ck1k + (inflagU)*ck2k;
-        const T Cout = (T(1) - inflagL) * ck1k + (T(1) - inflagU) * ck2k;
-        const T zerosw = T(0.5) - sign_half(tabs(Cout) - EPS);
-#pragma unroll
-        for (int b = 0; b < TB; ++b) {
-            const int bb = b < nb ? b : 0;
-            const T qkp1 = q[bb * ts + o + s];
-            const T Qin_minL = dmin(qk[b], qkm1[b]) + (T(1) - inflagL) * BIG;
-            const T Qin_minU = dmin(qk[b], qkp1) + (T(1) - inflagU) * BIG;
-            const T Qin_maxL = dmax(qk[b], qkm1[b]) - (T(1) - inflagL) * BIG;
-            const T Qin_maxU = dmax(qk[b], qkp1) - (T(1) - inflagU) * BIG;
-            const T qnext_min = dmin(dmin(Qin_minL, Qin_minU), qk[b]);
-            const T qnext_max = dmax(dmax(Qin_maxL, Qin_maxU), qk[b]);
-            T CQin_min, CQin_max;
-            if constexpr (POLE) {
-                CQin_max = (inflagL) * (ck1k * Qin_maxL) + (inflagU) * (ck2k * Qin_maxU);
-                CQin_min = (inflagL) * (ck1k * Qin_minL) + (inflagU) * (ck2k * Qin_minU);
-            } else {
-                CQin_min = (inflagL)*ck1k * Qin_minL + (inflagU)*ck2k * Qin_minU;
-                CQin_max = (inflagL)*ck1k * Qin_maxL + (inflagU)*ck2k * Qin_maxU;
-            }
-            const T Qmin_k = ((qk[b] - qnext_max) + qnext_max * (Cin + Cout - dk) - CQin_max) / (Cout + zerosw) *
-                                 (T(1) - zerosw) + qk[b] * zerosw;
-            const T Qmax_k = ((qk[b] - qnext_min) + qnext_min * (Cin + Cout - dk) - CQin_min) / (Cout + zerosw) *
-                                 (T(1) - zerosw) + qk[b] * zerosw;
-            if (k >= kb && b < nb) {  // VLIM:179-180
-                const T qh = q_h[b * ts + o];
-                const T out = (inflagL)*dmax(dmin(qh, Qmax_km1[b]), Qmin_km1[b]) +
-                              (T(1) - inflagL) * dmax(dmin(qh, Qmax_k), Qmin_k);
-                stream_store(&q_h[b * ts + o], out);
-            }
-            Qmin_km1[b] = Qmin_k;
-            Qmax_km1[b] = Qmax_k;
-            qkm1[b] = qk[b];
-            qk[b] = qkp1;
-        }
-        ck1k = ck1kp1;
-    }
-}
-
-constexpr int VTB = 4;  // tracers per work-item in the batched kernel
-
-// the batched kernel: work-group = BLOCK columns at one run for one group of
-// VTB tracers; the tracer groups of one column block and run are neighbours
-template <class T>
-__device__ __forceinline__ void vlim_multi_block(const VlimArgs<T> &A, long blk)
+// A work-group is BLOCK consecutive columns at one run of levels for one
+// tracer.  The tracers and runs of one column block are consecutive
+// work-groups on one XCD: the tracers read the same ck and d, and each run
+// also reads the two levels below it, which the run below has just brought
+// into that XCD's L2.  Each XCD takes WIN column blocks at a time, next to the
+// other XCDs' (xcd_windowed): 154 us at gl7 FP64 against 163 us with an eighth
+// of the launch to each XCD; eight FP32 tracers on four grids 1.15 ms against
+// 1.25 ms with four tracers per work-item and their levels loaded one at a
+// time.  KC > 0: runs of KC levels known at compile time
+// (vlim_run_kc); 0: of A.kc levels (vlim_run; MASK only here).
+template <class T, int KC, bool MASK = false>
+__device__ __forceinline__ void vlim_block(const VlimArgs<T> &A, long blk)
 {
     const long ncol_reg = (long)A.gall * A.lall;
     const long ncol = ncol_reg + (A.have_pl ? (long)A.gall_pl * kLallPl : 0);
-    const long ncb = (ncol + BLOCK - 1) / BLOCK;
-    const int ngrp = (A.ntr + VTB - 1) / VTB;
-    const long L = xcd_contiguous(blk, ncb * A.nrun * ngrp);
-    const int grp = (int)(L % ngrp);
-    const int run = (int)((L / ngrp) % A.nrun);
-    const long col = (L / ngrp / A.nrun) * BLOCK + threadIdx.x;
+    const long ncb = (ncol + BLOCK - 1) / BLOCK;  // column blocks
+    const int unit = A.nrun * A.ntr;
+    const long L = xcd_windowed(blk, ncb * unit, WIN * unit);
+    const long cb = L / unit;
+    const int ru = (int)(L - cb * unit), run = ru / A.ntr, tr = ru - run * A.ntr;
+    const long col = cb * BLOCK + threadIdx.x;
     if (col >= ncol) return;
-    const int kmin = 1, kmax = A.kall - 2;
-    const int kb = kmin + 1 + run * A.kc;
-    const int ke = min(kmax + 1, kb + A.kc);
+    const int kmin = 1, kmax = A.kall - 2;  // 0-based
+    const int kc = KC > 0 ? KC : A.kc;
+    const int kb = kmin + 1 + run * kc;
+    const int ke = min(kmax + 1, kb + kc);
     if (kb >= ke) return;
-    const int t0 = grp * VTB, nb = min(VTB, A.ntr - t0);
-    if (col < ncol_reg) {
-        const int g = (int)(col % A.gall), l = (int)(col / A.gall);
-        const size_t base = (size_t)l * A.kall * A.gall + g;
-        const size_t ck2 = (size_t)A.gall * A.kall * A.lall;
-        vlim_run_multi<false, VTB, T>(A.q_h + t0 * A.ts, A.q + t0 * A.ts, A.d, A.ck, base, A.gall, ck2, kb, ke,
-                                      A.eps, A.big, nb, A.ts);
-    } else {
-        const int p = (int)(col - ncol_reg);
-        const int g = p % A.gall_pl, l = p / A.gall_pl;
-        const size_t base = (size_t)l * A.kall * A.gall_pl + g;
-        const size_t ck2 = (size_t)A.gall_pl * A.kall * kLallPl;
-        vlim_run_multi<true, VTB, T>(A.q_h_pl + t0 * A.tps, A.q_pl + t0 * A.tps, A.d_pl, A.ck_pl, base, A.gall_pl,
-                                     ck2, kb, ke, A.eps, A.big, nb, A.tps);
-    }
+    auto go = [&](auto pole, T *q_h, const T *q, const T *d, const T *ck, long t, int gall, int lall, uint32_t *mask) {
+        constexpr bool POLE = decltype(pole)::value;
+        const int g = (int)(t % gall), l = (int)(t / gall);
+        const size_t base = (size_t)l * A.kall * gall + g;
+        const size_t ck2 = (size_t)gall * A.kall * lall;
+        if constexpr (KC > 0)
+            vlim_run_kc<POLE, T, KC>(q_h, q, d, ck, base, gall, ck2, kb, ke, A.eps, A.big);
+        else
+            vlim_run<POLE, T, MASK>(q_h, q, d, ck, base, gall, ck2, kb, ke, A.eps, A.big,
+                                    MASK ? mask + ((size_t)l * A.nrun + run) * gall + g : nullptr);
+    };
+    if (col < ncol_reg)
+        go(std::false_type{}, A.q_h + tr * A.ts, A.q + tr * A.ts, A.d, A.ck, col, A.gall, A.lall, A.mask);
+    else
+        go(std::true_type{}, A.q_h_pl + tr * A.tps, A.q_pl + tr * A.tps, A.d_pl, A.ck_pl, col - ncol_reg, A.gall_pl,
+           kLallPl, A.mask_pl);
 }
 
-template <class T>
-__global__ void __launch_bounds__(BLOCK) vlim_multi_kernel(VlimArgs<T> A)
+template <class T, int KC, bool MASK = false>
+__global__ void __launch_bounds__(BLOCK) vlim_kernel(VlimArgs<T> A)
 {
-    vlim_multi_block<T>(A, blockIdx.x);
+    vlim_block<T, KC, MASK>(A, blockIdx.x);
 }
 
 // several grids in one launch: work-groups [off[n], off[n+1]) belong to grid n
@@ -299,69 +242,8 @@ __global__ void __launch_bounds__(BLOCK) vlim_group_kernel(VlimGroup<T> G)
     const int b = blockIdx.x;
     int n = 0;
     while (n + 1 < G.n && b >= G.off[n + 1]) ++n;
-    vlim_multi_block<T>(G.a[n], b - G.off[n]);
-}
-
-// A work-group is BLOCK consecutive columns at one run of levels.  The runs
-// of one column block are consecutive work-groups on one XCD: each run also
-// reads the two levels below it, which the run below has just brought into L2.
-template <class T, bool MASK = false>
-__global__ void __launch_bounds__(BLOCK) vlim_kernel(VlimArgs<T> A)
-{
-    const long ncol_reg = (long)A.gall * A.lall;
-    const long ncol = ncol_reg + (A.have_pl ? (long)A.gall_pl * kLallPl : 0);
-    const long ncb = (ncol + BLOCK - 1) / BLOCK;  // column blocks
-    const long L = xcd_contiguous(blockIdx.x, ncb * A.nrun);
-    const int run = (int)(L % A.nrun);
-    const long col = (L / A.nrun) * BLOCK + threadIdx.x;
-    if (col >= ncol) return;
-    const int kmin = 1, kmax = A.kall - 2;  // 0-based
-    const int kb = kmin + 1 + run * A.kc;
-    const int ke = min(kmax + 1, kb + A.kc);
-    if (kb >= ke) return;
-    if (col < ncol_reg) {
-        const int g = (int)(col % A.gall), l = (int)(col / A.gall);
-        const size_t base = (size_t)l * A.kall * A.gall + g;
-        const size_t ck2 = (size_t)A.gall * A.kall * A.lall;
-        uint32_t *mw = MASK ? A.mask + ((size_t)l * A.nrun + run) * A.gall + g : nullptr;
-        vlim_run<false, T, MASK>(A.q_h, A.q, A.d, A.ck, base, A.gall, ck2, kb, ke, A.eps, A.big, mw);
-    } else {
-        const int p = (int)(col - ncol_reg);
-        const int g = p % A.gall_pl, l = p / A.gall_pl;
-        const size_t base = (size_t)l * A.kall * A.gall_pl + g;
-        const size_t ck2 = (size_t)A.gall_pl * A.kall * kLallPl;
-        uint32_t *mw = MASK ? A.mask_pl + ((size_t)l * A.nrun + run) * A.gall_pl + g : nullptr;
-        vlim_run<true, T, MASK>(A.q_h_pl, A.q_pl, A.d_pl, A.ck_pl, base, A.gall_pl, ck2, kb, ke, A.eps, A.big, mw);
-    }
-}
-
-// vlim_kernel with KC-level runs (vlim_run_kc); no mask.
-template <class T, int KC>
-__global__ void __launch_bounds__(BLOCK) vlim_kernel_kc(VlimArgs<T> A)
-{
-    const long ncol_reg = (long)A.gall * A.lall;
-    const long ncol = ncol_reg + (A.have_pl ? (long)A.gall_pl * kLallPl : 0);
-    const long ncb = (ncol + BLOCK - 1) / BLOCK;  // column blocks
-    const long L = xcd_contiguous(blockIdx.x, ncb * A.nrun);
-    const int run = (int)(L % A.nrun);
-    const long col = (L / A.nrun) * BLOCK + threadIdx.x;
-    if (col >= ncol) return;
-    const int kmin = 1, kmax = A.kall - 2;  // 0-based
-    const int kb = kmin + 1 + run * KC;
-    const int ke = min(kmax + 1, kb + KC);
-    if (kb >= ke) return;
-    if (col < ncol_reg) {
-        const int g = (int)(col % A.gall), l = (int)(col / A.gall);
-        const size_t base = (size_t)l * A.kall * A.gall + g;
-        const size_t ck2 = (size_t)A.gall * A.kall * A.lall;
-        vlim_run_kc<false, T, KC>(A.q_h, A.q, A.d, A.ck, base, A.gall, ck2, kb, ke, A.eps, A.big);
-    } else {
-        const int p = (int)(col - ncol_reg);
-        const int g = p % A.gall_pl, l = p / A.gall_pl;
-        const size_t base = (size_t)l * A.kall * A.gall_pl + g;
-        const size_t ck2 = (size_t)A.gall_pl * A.kall * kLallPl;
-        vlim_run_kc<true, T, KC>(A.q_h_pl, A.q_pl, A.d_pl, A.ck_pl, base, A.gall_pl, ck2, kb, ke, A.eps, A.big);
-    }
+    if (G.a[n].kc == RUN_KC) vlim_block<T, RUN_KC>(G.a[n], b - G.off[n]);
+    else vlim_block<T, 0>(G.a[n], b - G.off[n]);  // a run length chosen by tuning
 }
 
 }  // namespace
@@ -371,7 +253,7 @@ namespace {
 template <class T>
 int vlim_make_args(nicam_ctx c, VlimArgs<T> &A, long &nblk, T *q_h, T *q_h_pl, const T *q, const T *q_pl,
                    const T *d, const T *d_pl, const T *ck, const T *ck_pl, T eps, T big, uint32_t *mask,
-                   uint32_t *mask_pl, int ntr, bool multi)
+                   uint32_t *mask_pl, int ntr)
 {
     const Dims &D = c->d;
     if (ntr < 1 || (mask && ntr != 1)) return fail(NICAM_ERR_ARG, "tracer count must be >= 1 (1 with a mask)");
@@ -398,15 +280,14 @@ int vlim_make_args(nicam_ctx c, VlimArgs<T> &A, long &nblk, T *q_h, T *q_h_pl, c
     nblk = 0;
     const int nlev = D.kall - 3;  // limited levels kmin+1..kmax
     if (nlev <= 0) return NICAM_OK;
-    // runtime-length runs: short runs give more independent work-items (measured best at gl7: 4); the
-    // single-tracer kernel without a mask takes compile-time runs of NICAM_VLIM_KC levels instead
-    int kc = c->tune.vlim_kchunk > 0 ? c->tune.vlim_kchunk : (!multi && !mask && NICAM_VLIM_KC > 0 ? NICAM_VLIM_KC : 4);
+    // short runs give more independent work-items; other lengths than RUN_KC are runtime-length runs
+    int kc = c->tune.vlim_kchunk > 0 ? c->tune.vlim_kchunk : RUN_KC;
     if (mask) kc = 32;  // one mask word per run
-    kc = std::min(kc, nlev);
+    if (kc != RUN_KC) kc = std::min(kc, nlev);
     A.kc = kc;
     A.nrun = (nlev + kc - 1) / kc;
     const long ncol = (long)D.gall * D.lall + (D.have_pl ? (long)D.gall_pl * kLallPl : 0);
-    nblk = (ncol + BLOCK - 1) / BLOCK * A.nrun * (multi ? (ntr + VTB - 1) / VTB : 1);
+    nblk = (ncol + BLOCK - 1) / BLOCK * A.nrun * ntr;
     if (nblk > 0x7fffffffL) return fail(NICAM_ERR_ARG, "grid too large for one launch");
     return NICAM_OK;
 }
@@ -418,16 +299,12 @@ int launch_vlim_t(nicam_ctx c, T *q_h, T *q_h_pl, const T *q, const T *q_pl, con
 {
     VlimArgs<T> A;
     long nblk = 0;
-    const int rc = vlim_make_args(c, A, nblk, q_h, q_h_pl, q, q_pl, d, d_pl, ck, ck_pl, eps, big, mask, mask_pl, ntr,
-                                  ntr > 1);
+    const int rc = vlim_make_args(c, A, nblk, q_h, q_h_pl, q, q_pl, d, d_pl, ck, ck_pl, eps, big, mask, mask_pl, ntr);
     if (rc != NICAM_OK || nblk == 0) return rc;
-    if (ntr > 1)
-        hipLaunchKernelGGL(vlim_multi_kernel<T>, dim3((unsigned)nblk), dim3(BLOCK), 0, c->stream, A);
-    else if (mask) hipLaunchKernelGGL((vlim_kernel<T, true>), dim3((unsigned)nblk), dim3(BLOCK), 0, c->stream, A);
-    else if (NICAM_VLIM_KC > 0 && A.kc == NICAM_VLIM_KC)
-        hipLaunchKernelGGL((vlim_kernel_kc<T, (NICAM_VLIM_KC > 0 ? NICAM_VLIM_KC : 1)>), dim3((unsigned)nblk),
-                           dim3(BLOCK), 0, c->stream, A);
-    else hipLaunchKernelGGL((vlim_kernel<T, false>), dim3((unsigned)nblk), dim3(BLOCK), 0, c->stream, A);
+    const dim3 grid((unsigned)nblk), blk(BLOCK);
+    if (mask) hipLaunchKernelGGL((vlim_kernel<T, 0, true>), grid, blk, 0, c->stream, A);
+    else if (A.kc == RUN_KC) hipLaunchKernelGGL((vlim_kernel<T, RUN_KC>), grid, blk, 0, c->stream, A);
+    else hipLaunchKernelGGL((vlim_kernel<T, 0>), grid, blk, 0, c->stream, A);
     NICAM_HIP(hipGetLastError());
     return NICAM_OK;
 }
@@ -485,7 +362,7 @@ int launch_vlim_group_f32(const nicam_ctx *cs, int n, int ntr, const nicam_trace
         const nicam_tracer_step_f32 &p = g[i];
         long nb = 0;
         const int rc = vlim_make_args<float>(cs[i], G.a[i], nb, p.q_h, p.q_h_pl, p.qv, p.qv_pl, p.dv, p.dv_pl, p.ck,
-                                             p.ck_pl, cs[i]->eps32, cs[i]->big32, nullptr, nullptr, ntr, true);
+                                             p.ck_pl, cs[i]->eps32, cs[i]->big32, nullptr, nullptr, ntr);
         if (rc != NICAM_OK) return rc;
         if ((long)G.off[i] + nb > 0x7fffffffL) return fail(NICAM_ERR_ARG, "group too large for one launch");
         G.off[i + 1] = G.off[i] + (int)nb;

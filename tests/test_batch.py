@@ -99,6 +99,31 @@ def test_gpu_batched_limiters_equal_single_tracer_calls(gpu, single, grid):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("ntr,kall,kc", [(3, 10, 0), (1, 11, 0), (2, 9, 3), (3, 4, 0)])
+def test_gpu_batched_vertical_limiter_maps_every_work_group(gpu, oracle, ntr, kall, kc):
+    """Enough column blocks (182 with the poles) for several full windows of
+    the XCD mapping and a remainder, every tracer against the oracle."""
+    import torch
+
+    spec = synth.GridSpec(34, kall, 40, have_pl=True, seed=66)
+    case = synth.make_case(spec, have_sgp=[1] + [0] * 39)
+    ctx = drivers.setup_context(spec, case["geo"])
+    ctx.set_tuning(runtime.TUNE_VLIM_KCHUNK, kc)
+    up = lambda x: torch.from_numpy(np.ascontiguousarray(x)).to(gpu)  # noqa: E731
+    vs = [dict(case["vlim"], q=np.roll(case["vlim"]["q"], 7 * t, -1), q_h=np.roll(case["vlim"]["q_h"], 3 * t, -1))
+          for t in range(ntr)]
+    st = {k: up(np.stack([v[k] for v in vs])) for k in ("q", "q_pl", "q_h", "q_h_pl")}
+    v = {k: up(vs[0][k]) for k in ("d", "d_pl", "ck", "ck_pl")}
+    ctx.vertical_limiter_thuburn_batch(ntr, st["q_h"], st["q_h_pl"], st["q"], st["q_pl"], v["d"], v["d_pl"], v["ck"],
+                                       v["ck_pl"])
+    for t in range(ntr):
+        want = oracle.vertical_limiter_thuburn(spec, vs[t])
+        for k in ("q_h", "q_h_pl"):
+            assert np.array_equal(st[k][t].cpu().numpy(), want[k]), (t, k)
+    ctx.close()
+
+
+@pytest.mark.gpu
 def test_gpu_batched_limiter_with_library_exchange(gpu):
     """Qout_post = NULL: the exchange runs on every tracer's Qout at once."""
     import torch
