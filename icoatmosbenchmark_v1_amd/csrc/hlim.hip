@@ -49,10 +49,6 @@ __device__ __forceinline__ T ld_once(const T *p)
 #endif
 }
 
-template <class T>
-__device__ __forceinline__ T dmin(T a, T b) { return (b < a) ? b : a; }
-template <class T>
-__device__ __forceinline__ T dmax(T a, T b) { return (b > a) ? b : a; }
 // Fortran SIGN(0.5, x): 0.5 with the sign bit of x
 __device__ __forceinline__ double sign_half(double x) { return copysign(0.5, x); }
 __device__ __forceinline__ float sign_half(float x) { return copysignf(0.5f, x); }
@@ -150,7 +146,7 @@ __device__ __forceinline__ void hlim_block(const HlimArgs<T> &A, int b)
 #pragma unroll
         for (int f = 0; f < 6; ++f) {
             chv[f] = ld_once(&A.ch[(size_t)f * plane + fb + g]);
-            chm[f] = dmin(chv[f], T(0));
+            chm[f] = hw_min(chv[f], T(0));
         }
         Cin_sum = chm[0] + chm[1] + chm[2] + chm[3] + chm[4] + chm[5];
         Cout_sum = chv[0] - chm[0] + chv[1] - chm[1] + chv[2] - chm[2] + chv[3] - chm[3] + chv[4] - chm[4] +
@@ -242,14 +238,19 @@ __device__ __forceinline__ void hlim_block(const HlimArgs<T> &A, int b)
                 const int im1j = max(p - 1, 0);
                 a = Q(p); b2 = Q(p + iall + 1); c2 = Q(p + iall); d2 = Q(im1j);
             }
-            qmn = dmin(dmin(dmin(a, b2), c2), d2);
-            qmx = dmax(dmax(dmax(a, b2), c2), d2);
+            qmn = keep_nan(a, hw_min(hw_min3(a, b2, c2), d2));
+            qmx = keep_nan(a, hw_max(hw_max3(a, b2, c2), d2));
         };
 
-        T omn[3], omx[3];
+        T omn[3], omx[3], in_mn_s[3], in_mx_s[3];  // own arcs: min/max and the bounds on their own side (:162-187)
         if (own) {
 #pragma unroll
-            for (int m = 0; m < 3; ++m) arc_minmax(m, g, omn[m], omx[m]);
+            for (int m = 0; m < 3; ++m) {
+                const T c = ocm[m];
+                arc_minmax(m, g, omn[m], omx[m]);
+                in_mn_s[m] = (c)*omn[m] + (T(1) - c) * BIG;
+                in_mx_s[m] = (c)*omx[m] + (T(1) - c) * (-BIG);
+            }
         }
 
         // ---- phase 1: allowable range of the cell (HLIM:216-301) ----
@@ -259,10 +260,9 @@ __device__ __forceinline__ void hlim_block(const HlimArgs<T> &A, int b)
         if (p1) {
             T qinmn[6], qinmx[6];
 #pragma unroll
-            for (int m = 0; m < 3; ++m) {  // faces 1..3: own side of own arcs (:162-187)
-                const T c = ocm[m];
-                qinmn[m] = (c)*omn[m] + (T(1) - c) * BIG;
-                qinmx[m] = (c)*omx[m] + (T(1) - c) * (-BIG);
+            for (int m = 0; m < 3; ++m) {  // faces 1..3
+                qinmn[m] = in_mn_s[m];
+                qinmx[m] = in_mx_s[m];
             }
             // faces 4..6: neighbour side of the arcs at (i-1,j), (i-1,j-1), (i,j-1)
 #pragma unroll
@@ -275,9 +275,10 @@ __device__ __forceinline__ void hlim_block(const HlimArgs<T> &A, int b)
             }
             T qnext_min = qc, qnext_max = qc;
 #pragma unroll
-            for (int f = 0; f < 6; ++f) qnext_min = dmin(qnext_min, qinmn[f]);
-#pragma unroll
-            for (int f = 0; f < 6; ++f) qnext_max = dmax(qnext_max, qinmx[f]);
+            for (int f = 0; f < 6; f += 2) {
+                qnext_min = hw_min3(qnext_min, qinmn[f], qinmn[f + 1]);
+                qnext_max = hw_max3(qnext_max, qinmx[f], qinmx[f + 1]);
+            }
             const T CQin_min_sum = chm[0] * qinmn[0] + chm[1] * qinmn[1] + chm[2] * qinmn[2] +
                                    chm[3] * qinmn[3] + chm[4] * qinmn[4] + chm[5] * qinmn[5];
             const T CQin_max_sum = chm[0] * qinmx[0] + chm[1] * qinmx[1] + chm[2] * qinmx[2] +
@@ -310,16 +311,15 @@ __device__ __forceinline__ void hlim_block(const HlimArgs<T> &A, int b)
 #pragma unroll
             for (int m = 0; m < 3; ++m) {
                 const T c = ocm[m];
-                const T in_mn_s = (c)*omn[m] + (T(1) - c) * BIG;
-                const T in_mx_s = (c)*omx[m] + (T(1) - c) * (-BIG);
                 const T in_mn_n = (c)*BIG + (T(1) - c) * omn[m];
                 const T in_mx_n = (c) * (-BIG) + (T(1) - c) * omx[m];
                 const T qo_min_n = PF ? pre_qpn[m][0] : Qpost[fb + nb[m]];
                 const T qo_max_n = PF ? pre_qpn[m][1] : Qpost[plane + fb + nb[m]];
                 T qa = PF ? pre_qa[m] : ld_once(&q_a[(size_t)m * plane + fb + g]);
                 const T qa_in = qa;
-                qa = (c)*dmin(dmax(qa, in_mn_s), in_mx_s) + (T(1) - c) * dmin(dmax(qa, in_mn_n), in_mx_n);
-                qa = (c)*dmax(dmin(qa, qo_max_n), qo_min_n) + (T(1) - c) * dmax(dmin(qa, qo_max_c), qo_min_c);
+                qa = (c)*hw_min(hw_max(qa, in_mn_s[m]), in_mx_s[m]) + (T(1) - c) * hw_min(hw_max(qa, in_mn_n), in_mx_n);
+                qa = (c)*hw_max(hw_min(qa, qo_max_n), qo_min_n) + (T(1) - c) * hw_max(hw_min(qa, qo_max_c), qo_min_c);
+                qa = keep_nan(qa_in, qa);
                 bits |= (qa != qa_in ? 1u : 0u) << m;
 #if NICAM_HLIM_STORE == 2
                 q_a[(size_t)m * plane + fb + g] = qa;
@@ -392,8 +392,8 @@ __device__ void hlim_pole(const HlimArgs<T> &A0, int t, int tr)
         if (vp1 == npl) vp1 = 1;
         if (vm1 == 0) vm1 = npl - 1;
         const T a = A.q_pl[fb + 0], b = A.q_pl[fb + v], c2 = A.q_pl[fb + vm1], d2 = A.q_pl[fb + vp1];
-        const T mn = dmin(dmin(dmin(a, b), c2), d2);
-        const T mx = dmax(dmax(dmax(a, b), c2), d2);
+        const T mn = keep_nan(a, hw_min(hw_min3(a, b, c2), d2));
+        const T mx = keep_nan(a, hw_max(hw_max3(a, b, c2), d2));
         const T c = A.cmask_pl[fb + v];
         mn1 = (c)*mn + (T(1) - c) * BIG;
         mn2 = (c)*BIG + (T(1) - c) * mn;
@@ -405,8 +405,8 @@ __device__ void hlim_pole(const HlimArgs<T> &A0, int t, int tr)
     for (int v = 1; v < npl; ++v) {
         T mn1, mn2, mx1, mx2;
         qin(v, mn1, mn2, mx1, mx2);
-        qnext_min = dmin(qnext_min, mn1);
-        qnext_max = dmax(qnext_max, mx1);
+        qnext_min = hw_min(qnext_min, mn1);
+        qnext_max = hw_max(qnext_max, mx1);
     }
     T Cin = T(0), Cout = T(0), CQmax = T(0), CQmin = T(0);
     for (int v = 1; v < npl; ++v) {
@@ -439,8 +439,9 @@ __device__ void hlim_pole(const HlimArgs<T> &A0, int t, int tr)
         const T c = A.cmask_pl[fb + v];
         T qa = A.q_a_pl[fb + v];
         const T qa_in = qa;
-        qa = (c)*dmin(dmax(qa, mn1), mx1) + (T(1) - c) * dmin(dmax(qa, mn2), mx2);
-        qa = (c)*dmax(dmin(qa, A.Qpost_pl[plane + fb + v]), A.Qpost_pl[fb + v]) + (T(1) - c) * dmax(dmin(qa, pn_max), pn_min);
+        qa = (c)*hw_min(hw_max(qa, mn1), mx1) + (T(1) - c) * hw_min(hw_max(qa, mn2), mx2);
+        qa = (c)*hw_max(hw_min(qa, A.Qpost_pl[plane + fb + v]), A.Qpost_pl[fb + v]) + (T(1) - c) * hw_max(hw_min(qa, pn_max), pn_min);
+        qa = keep_nan(qa_in, qa);
         A.q_a_pl[fb + v] = qa;
         if (A.mask_pl) A.mask_pl[fb + v] = (qa != qa_in) ? 1 : 0;
     }

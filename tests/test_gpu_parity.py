@@ -197,6 +197,31 @@ def test_hlim_variants(gpu, oracle, variant, c):
     assert_parity(got, want)
 
 
+@pytest.mark.parametrize("variant", [1, 2])
+@pytest.mark.parametrize("field", ["q", "q_a", "Qout_post", "ch", "d", "cmask"])
+def test_hlim_keeps_nan_and_infinity_where_the_reference_form_does(gpu, oracle, field, variant):
+    """NaN and infinities planted in each input: the limited faces and ranges
+    are NaN at exactly the oracle's places, and equal to it elsewhere."""
+    from icoatmosbenchmark_v1_amd.runtime import TUNE_HLIM_VARIANT
+
+    spec, case = _case(CASES[4])
+    h = {k: np.array(v) for k, v in case["hlim"].items()}
+    rng = np.random.default_rng(5)
+    for nm in (field, field + "_pl"):
+        flat = h[nm].reshape(-1)
+        for v in (np.nan, np.inf, -np.inf):
+            flat[rng.choice(flat.size, max(2, flat.size // 400), replace=False)] = v
+    ctx = drivers.setup_context(spec, case["geo"])
+    ctx.set_tuning(TUNE_HLIM_VARIANT, variant)
+    got = drivers.run_hlim(ctx, spec, h)
+    want = oracle.horizontal_limiter_thuburn(spec, case["geo"]["have_sgp"], h)
+    assert any(np.isnan(want[k]).any() for k in want)
+    for k in want:
+        if not spec.have_pl and k.endswith("_pl"):
+            continue
+        np.testing.assert_array_equal(got[k], want[k], err_msg=k)
+
+
 @pytest.mark.parametrize("kc", [1, 2, 5, 24, 1000])
 def test_vlim_level_runs(gpu, oracle, kc):
     spec, case = _case((10, 30, 2, 23, [0, 0], True))
