@@ -239,7 +239,7 @@ int nicam_ctx_set_tuning(nicam_ctx c, int param, int value)
     case NICAM_TUNE_DIFF_KPER: c->tune.diff_kper = value; break;
     case NICAM_TUNE_DDMP_KPER: c->tune.ddmp_kper = value; break;
     case NICAM_TUNE_VI_VARIANT:
-        if (value > 4) return fail(NICAM_ERR_ARG, "NICAM_TUNE_VI_VARIANT must be 0..4");
+        if (value > 5) return fail(NICAM_ERR_ARG, "NICAM_TUNE_VI_VARIANT must be 0..5");
         c->tune.vi_variant = value;
         break;
     case NICAM_TUNE_HLIM_VARIANT:

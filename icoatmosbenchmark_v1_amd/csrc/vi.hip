@@ -24,6 +24,9 @@
 //   3  unfactored, gamma and the forward solution in registers (fully
 //      unrolled levels; built for kall = 42 and 98)
 //   4  factored, forward solution in registers (kall = 42 and 98)
+//   5  factored, a work-group of four waves per 64 columns: the source term
+//      formed by all of them into LDS, the recurrences by the first (up to 320
+//      levels)
 // All of them produce the same bits: the factors are formed by the same
 // operations in the same order whether they are stored or not.
 #include <type_traits>
@@ -221,30 +224,6 @@ __global__ void __launch_bounds__(BLOCK_FAC) vi_kernel_fact(ViArgsT<Src> A)
     });
 }
 
-// several grids in one launch (factored, any kall): work-groups
-// [off[n], off[n+1]) belong to grid n
-template <class Src>
-struct ViGroup {
-    ViArgsT<Src> a[kMaxGroup];
-    int off[kMaxGroup + 1];
-    int n;
-};
-
-template <class Src>
-__global__ void __launch_bounds__(BLOCK_FAC) vi_group_kernel(ViGroup<Src> G)
-{
-    const int b = blockIdx.x;
-    int n = 0;
-    while (n + 1 < G.n && b >= G.off[n + 1]) ++n;
-    const ViArgsT<Src> &A = G.a[n];
-    column_run<BLOCK_FAC>(A, b - G.off[n], [&](const ViFieldT<Src> &F, size_t base, size_t s) {
-        NoGamma gam;
-        int unused = 0;
-        vi_column<0, false, true>(F, base, s, A.kall, A.rdgzh, A.afact, A.bfact, A.dt, A.CVovRt2, A.alpha, A.grav,
-                                  gam, unused);
-    });
-}
-
 template <int KC, bool FACT, class Src>
 __global__ void __launch_bounds__(BLOCK_REG) vi_kernel_reg(ViArgsT<Src> A)
 {
@@ -283,6 +262,189 @@ __global__ void __launch_bounds__(BLOCK_REG) vi_kernel_reg(ViArgsT<Src> A)
         column(*F, base, s);
     } else {
         column_run<BLOCK_REG>(A, xcd_contiguous(blockIdx.x, gridDim.x), column);  // FP32 sources: 309 us against 550 us per work-item
+    }
+}
+
+// Cooperative: a work-group of NW waves owns 64 columns.  The source term of
+// every level is independent of the others, so the waves form it together,
+// each on a contiguous range of levels with CB levels of loads in flight, into
+// LDS; the first wave then runs the two recurrences on LDS, with the factors
+// of the next CD levels in flight in registers; last, the waves scale and store
+// the solution together.  A column per work-item waits for memory once or more
+// per level, which only a grid of many thousands of columns hides, and its
+// chain of divisions stands behind those waits.  (At 40 x 66x66 x 97 with the
+// v-limiter: four waves 512 us, eight 589, four with two levels of loads 515.)
+constexpr int NW = 4, BLOCK_CO = 64 * NW;
+constexpr int CB = 4;   // levels of source loads in flight per wave
+constexpr int CD = 16;  // levels of factors in flight in the recurrences
+constexpr int CG = 16;  // levels of the final scaling in flight per wave
+
+template <class Src>
+__device__ __forceinline__ void vi_coop_block(const ViArgsT<Src> &A, long blk, double *s_w)
+{
+    const int kall = A.kall, kmin = 1, kmax = kall - 2;  // 0-based
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const long nreg = (long)A.gall * A.lall, nbr = (nreg + 63) / 64;
+    const bool reg = blk < nbr;
+    const ViFieldT<Src> &F = reg ? A.reg : A.pl;
+    const int gall = reg ? A.gall : A.gall_pl;
+    const long ncol = reg ? nreg : (long)A.gall_pl * kLallPl;
+    const long t0 = (reg ? blk : blk - nbr) * 64 + lane;
+    const bool have = t0 < ncol;  // lanes past the end work on the last column and store nothing
+    const long t = have ? t0 : ncol - 1;
+    const size_t base = (size_t)(t / gall) * kall * gall + (size_t)(t % gall), s = gall;
+    auto at = [&](int k) { return base + (size_t)k * s; };
+    auto W = [&](int k) -> double & { return s_w[(size_t)k * 64 + lane]; };
+    const double dt = A.dt, CV = A.CVovRt2, alpha = A.alpha, grav = A.grav;
+
+    const int nl = kmax - kmin, per = (nl + NW - 1) / NW;  // levels kmin+1..kmax over the waves
+    const int ka = kmin + 1 + wv * per, ke = min(kmax + 1, ka + per);
+    // ---- the source term (mod_vi.f90:192-212) ----
+    if (ka < ke) {
+        double P_km1, R_km1;
+        {
+            const size_t o = at(ka - 1);
+            const double rg = F.RGAM[o];
+            P_km1 = (F.p0[o] + dt * F.Sp[o]) * F.RGSGAM2[o];
+            R_km1 = (F.r0[o] + dt * F.Sr[o]) * (rg * rg);
+        }
+        for (int kb = ka; kb < ke; kb += CB) {
+            Src rgh[CB], rg[CB], p0[CB], Sp[CB], rgs[CB], r0[CB], Sr[CB], w0[CB], Sw[CB];
+#pragma unroll
+            for (int c = 0; c < CB; ++c) {
+                const size_t o = at(min(kb + c, ke - 1));
+                rgh[c] = F.RGAMH[o];
+                rg[c] = F.RGAM[o];
+                p0[c] = F.p0[o];
+                Sp[c] = F.Sp[o];
+                rgs[c] = F.RGSGAM2[o];
+                r0[c] = F.r0[o];
+                Sr[c] = F.Sr[o];
+                w0[c] = F.w0[o];
+                Sw[c] = F.Sw[o];
+            }
+#pragma unroll
+            for (int c = 0; c < CB; ++c) {
+                const int k = kb + c;
+                if (k >= ke) break;
+                const double rgd = rg[c], rghd = rgh[c];
+                const double P_k = (p0[c] + dt * Sp[c]) * rgs[c];
+                const double R_k = (r0[c] + dt * Sr[c]) * (rgd * rgd);
+                double S = ((w0[c] * alpha + dt * Sw[c]) * (rghd * rghd) - (P_k - P_km1) * dt * A.rdgzh[k] -
+                            (R_k * A.afact[k] + R_km1 * A.bfact[k]) * dt * grav) *
+                           CV;
+                if (k == kmin + 1) S = S - F.Ml[at(k)] * (F.w[at(kmin)] * F.RGSGAM2H[at(kmin)]);  // :209, :211
+                if (k == kmax) S = S - F.Mu[at(k)] * (F.w[at(kmax + 1)] * F.RGSGAM2H[at(kmax + 1)]);  // :210, :212
+                W(k) = S;
+                P_km1 = P_k;
+                R_km1 = R_k;
+            }
+        }
+    }
+    // ---- the recurrences, in the first wave ----
+    double ml[CD], be[CD];
+    if (wv == 0) {
+#pragma unroll
+        for (int c = 0; c < CD; ++c) {
+            const size_t o = at(min(kmin + 1 + c, kmax));
+            ml[c] = F.Ml[o];
+            be[c] = F.beta[o];
+        }
+    }
+    __syncthreads();
+    if (wv == 0) {
+        double w = 0.0;
+        double sv[CD];
+        for (int kb = kmin + 1; kb <= kmax; kb += CD) {  // mod_vi.f90:218-231 with beta(k) stored
+#pragma unroll
+            for (int c = 0; c < CD; ++c) sv[c] = W(min(kb + c, kmax));
+#pragma unroll
+            for (int c = 0; c < CD; ++c) {
+                const int k = kb + c;
+                if (k <= kmax) {
+                    w = (k == kmin + 1 ? sv[c] : sv[c] - ml[c] * w) / be[c];
+                    W(k) = w;
+                }
+                const size_t o = at(min(k + CD, kmax));
+                ml[c] = F.Ml[o];
+                be[c] = F.beta[o];
+            }
+        }
+        double g[CD];
+#pragma unroll
+        for (int c = 0; c < CD; ++c) g[c] = F.gam[at(max(kmax - c, kmin + 1))];
+        for (int kb = kmax - 1; kb >= kmin + 1; kb -= CD) {  // mod_vi.f90:234-239
+#pragma unroll
+            for (int c = 0; c < CD; ++c) sv[c] = W(max(kb - c, kmin + 1));
+#pragma unroll
+            for (int c = 0; c < CD; ++c) {
+                const int k = kb - c;
+                if (k >= kmin + 1) {
+                    w = sv[c] - g[c] * w;
+                    W(k) = w;
+                }
+                g[c] = F.gam[at(max(k + 1 - CD, kmin + 1))];
+            }
+        }
+    }
+    // ---- scaled and stored (mod_vi.f90:242-246) ----
+    double gs[CG];
+    auto load_gs = [&](int kb) {
+#pragma unroll
+        for (int c = 0; c < CG; ++c) gs[c] = F.GSGAM2H[at(min(kb + c, kmax))];
+    };
+    load_gs(ka);
+    __syncthreads();
+    if (!have) return;
+    for (int kb = ka; kb < ke; kb += CG) {
+#pragma unroll
+        for (int c = 0; c < CG; ++c)
+            if (kb + c < ke) stream_store(&F.w[at(kb + c)], W(kb + c) * gs[c]);
+        if (kb + CG < ke) load_gs(kb + CG);
+    }
+    if (wv == NW - 1) {  // the boundary levels, scaled by both metrics in the reference's order
+        for (int k : {kmin, kmax + 1}) {
+            const double wb = F.w[at(k)] * F.RGSGAM2H[at(k)];
+            F.w[at(k)] = wb * F.GSGAM2H[at(k)];
+        }
+    }
+}
+
+template <class Src>
+__global__ void __launch_bounds__(BLOCK_CO) vi_kernel_coop(ViArgsT<Src> A)
+{
+    extern __shared__ double s_w[];
+    vi_coop_block<Src>(A, blockIdx.x, s_w);
+}
+
+static_assert(BLOCK_CO == 256 && BLOCK_FAC == 256, "vi_group_kernel serves both");
+
+// several grids in one launch (cooperative, or a column per work-item): work-groups
+// [off[n], off[n+1]) belong to grid n
+template <class Src>
+struct ViGroup {
+    ViArgsT<Src> a[kMaxGroup];
+    int off[kMaxGroup + 1];
+    int n;
+};
+
+template <class Src, bool COOP>
+__global__ void __launch_bounds__(256) vi_group_kernel(ViGroup<Src> G)
+{
+    const int b = blockIdx.x;
+    int n = 0;
+    while (n + 1 < G.n && b >= G.off[n + 1]) ++n;
+    const ViArgsT<Src> &A = G.a[n];
+    if constexpr (COOP) {
+        extern __shared__ double s_w[];
+        vi_coop_block<Src>(A, b - G.off[n], s_w);
+    } else {
+        column_run<BLOCK_FAC>(A, b - G.off[n], [&](const ViFieldT<Src> &F, size_t base, size_t s) {
+            NoGamma gam;
+            int unused = 0;
+            vi_column<0, false, true>(F, base, s, A.kall, A.rdgzh, A.afact, A.bfact, A.dt, A.CVovRt2, A.alpha, A.grav,
+                                      gam, unused);
+        });
     }
 }
 
@@ -334,6 +496,9 @@ __global__ void __launch_bounds__(BLOCK_FAC) vi_factor_kernel(FactorArgs A)
     }
 }
 
+constexpr int kMaxCoop = 320;  // levels whose column values fit 160 KiB of LDS
+size_t coop_lds(int kall) { return sizeof(double) * 64 * kall; }
+
 template <class Src>
 void vi_make_args(nicam_ctx c, ViArgsT<Src> &A, double *w, double *w_pl, const Src *w0, const Src *w0_pl,
                   const Src *p0, const Src *p0_pl, const Src *r0, const Src *r0_pl, const Src *Sr, const Src *Sr_pl,
@@ -374,10 +539,12 @@ int launch_vi_t(nicam_ctx c, double *w, double *w_pl, const Src *w0, const Src *
 
     int variant = c->tune.vi_variant;
     const bool reg_ok = (D.kall == 42 || D.kall == 98);
-    if ((variant == 3 || variant == 4) && !reg_ok) variant = 0;
-    // measured at gl7 (40 x 66x66 x 98): FP64 inputs: 4 (factored, registers) 368 us, 3 379, 2 469, 1 623;
-    // FP32 inputs: 4 309 us, 2 (factored, through rhogw) 324, 3 759, 1 633
-    if (variant == 0) variant = reg_ok ? 4 : 2;
+    if (((variant == 3 || variant == 4) && !reg_ok) || (variant == 5 && D.kall > kMaxCoop)) variant = 0;
+    // measured with the v-limiter (us; 5 against the best other): 40 x 66x66 x 98 FP64 518 against 533 (4), FP32
+    // inputs 346 against 400 (4); x 97 FP64 512 against 640 (2); 40 x 34x34 x 58 93 against 123 (2); 7 x 51x51 x 61
+    // 57.6 against 98.7 (2); 12x12 x 98 31.3 against 32.6 (4).  At 42 levels the registers hold the column at two
+    // waves per SIMD and 4 is as fast or faster (130x130 37.3 against 38.7, 10 x 66x66 68.1 against 71.9).
+    if (variant == 0) variant = D.kall == 42 ? 4 : (D.kall <= kMaxCoop ? 5 : 2);
 
     if (variant == 1) {
         const size_t lds = sizeof(double) * BLOCK_LDS * D.kall;
@@ -387,6 +554,13 @@ int launch_vi_t(nicam_ctx c, double *w, double *w_pl, const Src *w0, const Src *
                                           (int)lds));
         hipLaunchKernelGGL(vi_kernel_lds<Src>, dim3((unsigned)column_blocks<BLOCK_LDS>(D.gall, D.lall, D.gall_pl, D.have_pl)),
                            dim3(BLOCK_LDS), lds, c->stream, A);
+    } else if (variant == 5) {
+        const size_t lds = coop_lds(D.kall);
+        if (lds > 64 * 1024)
+            NICAM_HIP(hipFuncSetAttribute((const void *)vi_kernel_coop<Src>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                          (int)lds));
+        hipLaunchKernelGGL(vi_kernel_coop<Src>, dim3((unsigned)column_blocks<64>(D.gall, D.lall, D.gall_pl, D.have_pl)),
+                           dim3(BLOCK_CO), lds, c->stream, A);
     } else if (variant == 2) {
         hipLaunchKernelGGL(vi_kernel_fact<Src>, dim3((unsigned)column_blocks<BLOCK_FAC>(D.gall, D.lall, D.gall_pl, D.have_pl)),
                            dim3(BLOCK_FAC), 0, c->stream, A);
@@ -447,17 +621,30 @@ int launch_vi_group_mixed(const nicam_ctx *cs, int n, const nicam_tracer_step_f3
     ViGroup<float> G;
     G.n = n;
     G.off[0] = 0;
+    int kmax = 0;
+    for (int i = 0; i < n; ++i) kmax = std::max(kmax, cs[i]->d.kall);
+    const bool coop = kmax <= kMaxCoop;
     for (int i = 0; i < n; ++i) {
         const nicam_ctx c = cs[i];
         const nicam_tracer_step_f32 &p = g[i];
         vi_make_args<float>(c, G.a[i], p.rhogw, p.rhogw_pl, p.rhogw0, p.rhogw0_pl, p.preg0, p.preg0_pl, p.rhog0,
                             p.rhog0_pl, p.Srho, p.Srho_pl, p.Sw, p.Sw_pl, p.Spre, p.Spre_pl, dt, c->RGAM32,
                             c->RGAM32_pl, c->RGAMH32, c->RGAMH32_pl, c->RGSGAM2_32, c->RGSGAM2_32_pl);
-        const long nb = column_blocks<BLOCK_FAC>(G.a[i].gall, G.a[i].lall, G.a[i].gall_pl, G.a[i].have_pl);
+        const ViArgsT<float> &a = G.a[i];
+        const long nb = coop ? column_blocks<64>(a.gall, a.lall, a.gall_pl, a.have_pl)
+                             : column_blocks<BLOCK_FAC>(a.gall, a.lall, a.gall_pl, a.have_pl);
         if ((long)G.off[i] + nb > 0x7fffffffL) return fail(NICAM_ERR_ARG, "group too large for one launch");
         G.off[i + 1] = G.off[i] + (int)nb;
     }
-    hipLaunchKernelGGL(vi_group_kernel<float>, dim3((unsigned)G.off[n]), dim3(BLOCK_FAC), 0, stream, G);
+    if (coop) {
+        const size_t lds = coop_lds(kmax);
+        if (lds > 64 * 1024)
+            NICAM_HIP(hipFuncSetAttribute((const void *)vi_group_kernel<float, true>,
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        hipLaunchKernelGGL((vi_group_kernel<float, true>), dim3((unsigned)G.off[n]), dim3(BLOCK_CO), lds, stream, G);
+    } else {
+        hipLaunchKernelGGL((vi_group_kernel<float, false>), dim3((unsigned)G.off[n]), dim3(BLOCK_FAC), 0, stream, G);
+    }
     NICAM_HIP(hipGetLastError());
     return NICAM_OK;
 }
