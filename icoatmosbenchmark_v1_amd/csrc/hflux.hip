@@ -363,6 +363,35 @@ int hflux_launch(void (*const k[4])(Arg), int v, long nblk, size_t lds, hipStrea
     return NICAM_OK;
 }
 
+// Levels per work-group for base chunks of kall levels each.  The chip runs
+// SLOTS work-groups at a time (two per CU in FP64, by registers; four in FP32),
+// and each pays about one and a half levels for its metrics, so a launch costs
+// rounds * (levels + 1.5): the least of that over all splits, the longer march
+// on a tie.  FP64, us at kper: one 130x130x42 region 46.6 at 1, 39 at 2, 36 at 3,
+// 39 at 4, 35 at 6 (one round), 39.6 at 8, 49 at 14; 40 regions of 18x18x42 43 at
+// 1, 36 at 4, 32 at 7 (one round), 43 at 14; 34x34x78 155 at 4, 144 at 8, 152 at
+// 13, 178 at 26; 66x66x98 596 at 25 and 49, 617 at 33, 713 at 98: the order the
+// cost gives, every time.  FP32 keeps more work-groups in flight and gains from
+// short marches at any size (66x66x98 399 at 98, 359 at 33, 332 at 10; 130x130x98
+// 1238 at 49, 1195 at 14), hence its cap.
+template <class T>
+int hflux_kper(long base, int kall)
+{
+    const long slots = sizeof(T) == 8 ? 512 : 1024;
+    const int cap = sizeof(T) == 8 ? kall : std::min(kall, 14);
+    int best = 1;
+    double cost = 0.0;
+    for (int kper = 1; kper <= cap; ++kper) {
+        const long n = base * ((kall + kper - 1) / kper);
+        const double t = (double)((n + slots - 1) / slots) * (kper + 1.5);
+        if (kper == 1 || t <= cost) {
+            cost = t;
+            best = kper;
+        }
+    }
+    return best;
+}
+
 // The launch arguments of one grid: nblk work-groups, lds bytes, nst the
 // variant (hflux_variant) its width needs.
 template <class T>
@@ -390,12 +419,8 @@ int hflux_make_args(nicam_ctx c, HfluxArgs<T> &A, long &nblk, size_t &lds, int &
     A.dt = dt;
     A.eps = eps;
     A.nchunk = (D.gall + CHUNK - 1) / CHUNK;
-    // enough work-groups to fill 256 CUs several times over
     const long base = (long)A.nchunk * D.lall;
-    int nkr = (int)((4096 + base - 1) / base);
-    nkr = std::max(1, std::min(nkr, D.kall));
-    if (c->tune.hflux_kper > 0) nkr = (D.kall + c->tune.hflux_kper - 1) / c->tune.hflux_kper;
-    A.kper = (D.kall + nkr - 1) / nkr;
+    A.kper = c->tune.hflux_kper > 0 ? std::min(c->tune.hflux_kper, D.kall) : hflux_kper<T>(base, D.kall);
     A.nkr = (D.kall + A.kper - 1) / A.kper;
     const long nmain = base * A.nkr;
     const long npole = D.have_pl ? (D.kall * kLallPl + CHUNK - 1) / CHUNK : 0;
