@@ -25,6 +25,7 @@ namespace {
 
 constexpr int BLOCK = 256;
 constexpr int RUN_KC = 4;  // levels per run; gl7: 4 164 us, 8 168, 16 168, runtime-length 169 (FP64)
+constexpr int MASK_KC = 8; // faces per run of the masked kernel: a byte of a mask word
 constexpr int WIN = 4;     // column blocks an XCD takes at a time (gl7: 1 541 us for the vertical half, 4 530, 8 540)
 
 template <class T>
@@ -47,22 +48,18 @@ struct VlimArgs {
     T eps, big;
     int ntr;          // tracers
     long ts, tps;     // tracer strides of the regular and pole fields
-    uint32_t *mask, *mask_pl;  // clip bits (masked variant only; kc = 32)
+    uint32_t *mask, *mask_pl;  // clip bits (masked variant only; kc = 8)
 };
 
 // Levels [kb, ke) of one column are limited (kb >= kmin+1, 0-based).
 // base = offset of level 0, s = stride between levels, ck2 = offset of the
 // upper-face plane of ck.  POLE selects the pole loop's product grouping of
 // CQin (VLIM:212-215 versus :126-129).
-// MASK: also record one bit per limited face, set where the limited value
-// differs from q_h's input, in the word at mask_word (the run is the 32
-// faces of that word).
-template <bool POLE, class T, bool MASK = false>
+template <bool POLE, class T>
 __device__ __forceinline__ void vlim_run(T *__restrict__ q_h, const T *__restrict__ q, const T *__restrict__ d,
                                          const T *__restrict__ ck, size_t base, size_t s, size_t ck2, int kb,
-                                         int ke, T EPS, T BIG, uint32_t *mask_word = nullptr)
+                                         int ke, T EPS, T BIG)
 {
-    uint32_t bits = 0;
     int k = kb - 1;  // first level whose Qout is needed
     T qkm1 = q[base + (size_t)(k - 1) * s];
     T qk = q[base + (size_t)k * s];
@@ -101,7 +98,6 @@ __device__ __forceinline__ void vlim_run(T *__restrict__ q_h, const T *__restric
             const T qh = q_h[o];
             const T out = (inflagL)*dmax(dmin(qh, Qmax_km1), Qmin_km1) + (T(1) - inflagL) * dmax(dmin(qh, Qmax_k), Qmin_k);
             stream_store(&q_h[o], out);
-            if constexpr (MASK) bits |= (out != qh ? 1u : 0u) << (k - kb);
         }
         Qmin_km1 = Qmin_k;
         Qmax_km1 = Qmax_k;
@@ -109,7 +105,6 @@ __device__ __forceinline__ void vlim_run(T *__restrict__ q_h, const T *__restric
         qk = qkp1;
         ck1k = ck1kp1;
     }
-    if constexpr (MASK) *mask_word = bits;
 }
 
 // vlim_run with the run's length fixed at KC levels at compile time: every
@@ -119,9 +114,10 @@ __device__ __forceinline__ void vlim_run(T *__restrict__ q_h, const T *__restric
 // (fewer levels re-read at run edges) without losing loads in flight.  A
 // shorter last run (ke - kb < KC) reads level ke in place of the levels past
 // it and stores nothing there.  Same operations, in the same order, as
-// vlim_run.
+// vlim_run.  Returns a bit per face of the run, set where the limited value
+// differs from q_h's input (dead code unless the caller stores it).
 template <bool POLE, class T, int KC>
-__device__ __forceinline__ void vlim_run_kc(T *__restrict__ q_h, const T *__restrict__ q, const T *__restrict__ d,
+__device__ __forceinline__ uint32_t vlim_run_kc(T *__restrict__ q_h, const T *__restrict__ q, const T *__restrict__ d,
                                             const T *__restrict__ ck, size_t base, size_t s, size_t ck2, int kb,
                                             int ke, T EPS, T BIG)
 {
@@ -138,6 +134,7 @@ __device__ __forceinline__ void vlim_run_kc(T *__restrict__ q_h, const T *__rest
     }
 #pragma unroll
     for (int t = 0; t < KC; ++t) qh[t] = q_h[at(kb + t)];
+    uint32_t bits = 0;
     T Qmin_km1 = T(0), Qmax_km1 = T(0);
 #pragma unroll
     for (int t = 0; t <= KC; ++t) {  // level k = kb - 1 + t
@@ -171,10 +168,12 @@ __device__ __forceinline__ void vlim_run_kc(T *__restrict__ q_h, const T *__rest
             const T qhv = qh[t - 1];
             const T out = (inflagL)*dmax(dmin(qhv, Qmax_km1), Qmin_km1) + (T(1) - inflagL) * dmax(dmin(qhv, Qmax_k), Qmin_k);
             stream_store(&q_h[base + (size_t)k * s], out);
+            bits |= (out != qhv ? 1u : 0u) << (t - 1);
         }
         Qmin_km1 = Qmin_k;
         Qmax_km1 = Qmax_k;
     }
+    return bits;
 }
 
 // A work-group is BLOCK consecutive columns at one run of levels for one
@@ -186,7 +185,10 @@ __device__ __forceinline__ void vlim_run_kc(T *__restrict__ q_h, const T *__rest
 // of the launch to each XCD; eight FP32 tracers on four grids 1.15 ms against
 // 1.25 ms with four tracers per work-item and their levels loaded one at a
 // time.  KC > 0: runs of KC levels known at compile time
-// (vlim_run_kc); 0: of A.kc levels (vlim_run; MASK only here).
+// (vlim_run_kc); 0: of A.kc levels (vlim_run).
+// MASK: with runs of eight faces, a byte of the 32-face mask words each (face
+// p is bit p % 32 of word p / 32); the last run clears its word's other bytes.
+// (18x18x42x40, where runs of a whole word leave 102 work-groups: 58 -> 12 us.)
 template <class T, int KC, bool MASK = false>
 __device__ __forceinline__ void vlim_block(const VlimArgs<T> &A, long blk)
 {
@@ -209,11 +211,19 @@ __device__ __forceinline__ void vlim_block(const VlimArgs<T> &A, long blk)
         const int g = (int)(t % gall), l = (int)(t / gall);
         const size_t base = (size_t)l * A.kall * gall + g;
         const size_t ck2 = (size_t)gall * A.kall * lall;
-        if constexpr (KC > 0)
-            vlim_run_kc<POLE, T, KC>(q_h, q, d, ck, base, gall, ck2, kb, ke, A.eps, A.big);
-        else
-            vlim_run<POLE, T, MASK>(q_h, q, d, ck, base, gall, ck2, kb, ke, A.eps, A.big,
-                                    MASK ? mask + ((size_t)l * A.nrun + run) * gall + g : nullptr);
+        if constexpr (KC > 0) {
+            const uint32_t bits = vlim_run_kc<POLE, T, KC>(q_h, q, d, ck, base, gall, ck2, kb, ke, A.eps, A.big);
+            if constexpr (MASK) {
+                static_assert(KC == 8, "a run is one byte of a mask word");
+                const int nword = (A.nrun + 3) / 4;
+                uint8_t *byte = reinterpret_cast<uint8_t *>(mask + ((size_t)l * nword + run / 4) * gall + g);
+                byte[run % 4] = (uint8_t)bits;
+                if (run == A.nrun - 1)
+                    for (int r = run % 4 + 1; r < 4; ++r) byte[r] = 0;
+            }
+        } else {
+            vlim_run<POLE, T>(q_h, q, d, ck, base, gall, ck2, kb, ke, A.eps, A.big);
+        }
     };
     if (col < ncol_reg)
         go(std::false_type{}, A.q_h + tr * A.ts, A.q + tr * A.ts, A.d, A.ck, col, A.gall, A.lall, A.mask);
@@ -282,8 +292,8 @@ int vlim_make_args(nicam_ctx c, VlimArgs<T> &A, long &nblk, T *q_h, T *q_h_pl, c
     if (nlev <= 0) return NICAM_OK;
     // short runs give more independent work-items; other lengths than RUN_KC are runtime-length runs
     int kc = c->tune.vlim_kchunk > 0 ? c->tune.vlim_kchunk : RUN_KC;
-    if (mask) kc = 32;  // one mask word per run
-    if (kc != RUN_KC) kc = std::min(kc, nlev);
+    if (mask) kc = MASK_KC;
+    if (kc != RUN_KC && !mask) kc = std::min(kc, nlev);
     A.kc = kc;
     A.nrun = (nlev + kc - 1) / kc;
     const long ncol = (long)D.gall * D.lall + (D.have_pl ? (long)D.gall_pl * kLallPl : 0);
@@ -302,7 +312,7 @@ int launch_vlim_t(nicam_ctx c, T *q_h, T *q_h_pl, const T *q, const T *q_pl, con
     const int rc = vlim_make_args(c, A, nblk, q_h, q_h_pl, q, q_pl, d, d_pl, ck, ck_pl, eps, big, mask, mask_pl, ntr);
     if (rc != NICAM_OK || nblk == 0) return rc;
     const dim3 grid((unsigned)nblk), blk(BLOCK);
-    if (mask) hipLaunchKernelGGL((vlim_kernel<T, 0, true>), grid, blk, 0, c->stream, A);
+    if (mask) hipLaunchKernelGGL((vlim_kernel<T, MASK_KC, true>), grid, blk, 0, c->stream, A);
     else if (A.kc == RUN_KC) hipLaunchKernelGGL((vlim_kernel<T, RUN_KC>), grid, blk, 0, c->stream, A);
     else hipLaunchKernelGGL((vlim_kernel<T, 0>), grid, blk, 0, c->stream, A);
     NICAM_HIP(hipGetLastError());
