@@ -39,7 +39,7 @@ from typing import Dict, List, Sequence, Tuple
 import numpy as np
 import torch
 
-from .autodiff import RhowSolve, VerticalLimiter
+from .autodiff import RhowSolve
 from .drivers import VI_IN
 from .runtime import Context
 
@@ -50,8 +50,9 @@ class HorizontalFlux(torch.autograd.Function):
     @staticmethod
     def forward(fctx, nctx: Context, dt: float, *X):
         rho, rho_pl = X[0], X[1]
-        flx, flx_pl = rho.new_zeros((6,) + rho.shape), rho_pl.new_zeros(rho_pl.shape)
-        xc, xc_pl = rho.new_zeros((3, 3) + rho.shape), rho_pl.new_zeros((3,) + rho_pl.shape)
+        # the flux writes every face and centroid of the regions; a pole ring's centre stays zero
+        flx, flx_pl = rho.new_empty((6,) + rho.shape), rho_pl.new_zeros(rho_pl.shape)
+        xc, xc_pl = rho.new_empty((3, 3) + rho.shape), rho_pl.new_zeros((3,) + rho_pl.shape)
         nctx.horizontal_flux(flx, flx_pl, xc, xc_pl, *X, dt)
         fctx.nctx, fctx.dt = nctx, dt
         fctx.save_for_backward(*X)
@@ -69,44 +70,6 @@ class HorizontalFlux(torch.autograd.Function):
         b = [torch.empty_like(x) for x in X]
         fctx.nctx.horizontal_flux_adjoint(gf, gf_pl, gx, gx_pl, *b, *X, fctx.dt)
         return (None, None, *b)
-
-
-class HorizontalLimiter(torch.autograd.Function):
-    """q_a' = horizontal_limiter_thuburn(q_a, q, ch; d, cmask) (HLIM:42-430) in
-    the library's exchange mode: the allowable range Qout_prev, its halo
-    exchange (Qout_post) and the clamp, one masked call; d and cmask held fixed.
-    Its transpose: the faces' half pass of the limiter's adjoint (q_a_b ->
-    q_a's, q's and Qout_post's cotangents), the halo exchange's transpose
-    (Qout_post's -> Qout_prev's) and the rows' half pass (Qout_prev's -> q's and
-    ch's)."""
-
-    @staticmethod
-    def forward(fctx, nctx: Context, q_a, q_a_pl, q, q_pl, d, d_pl, ch, ch_pl, cm, cm_pl):
-        out, out_pl = q_a.clone(), q_a_pl.clone()
-        post, post_pl = q.new_zeros((2,) + q.shape), q_pl.new_zeros((2,) + q_pl.shape)
-        mask = torch.empty(q.shape, dtype=torch.uint8, device=q.device)
-        mask_pl = torch.empty(q_pl.shape, dtype=torch.uint8, device=q.device)
-        nctx.horizontal_limiter_thuburn_mask(out, out_pl, q, q_pl, d, d_pl, ch, ch_pl, cm, cm_pl, post, post_pl,
-                                             None, None, mask, mask_pl)
-        fctx.nctx = nctx
-        fctx.save_for_backward(out, out_pl, q, q_pl, post, post_pl, d, d_pl, ch, ch_pl, cm, cm_pl, mask, mask_pl)
-        return out, out_pl
-
-    @staticmethod
-    def backward(fctx, g_qa, g_qa_pl):
-        out, out_pl, q, q_pl, post, post_pl, d, d_pl, ch, ch_pl, cm, cm_pl, mask, mask_pl = fctx.saved_tensors
-        nctx = fctx.nctx
-        qab = torch.zeros_like(out) if g_qa is None else g_qa.contiguous().clone()
-        qab_pl = torch.zeros_like(out_pl) if g_qa_pl is None else g_qa_pl.contiguous().clone()
-        qb, qb_pl = torch.empty_like(q), torch.empty_like(q_pl)
-        pb, pb_pl = torch.empty_like(post), torch.empty_like(post_pl)
-        fixed = (out, out_pl, q, q_pl, d, d_pl, ch, ch_pl, cm, cm_pl, post, post_pl, mask, mask_pl)
-        nctx.horizontal_limiter_thuburn_adjoint(qab, qab_pl, qb, qb_pl, None, None, pb, pb_pl, *fixed)
-        nctx.comm_data_transfer_adjoint(pb, pb_pl, vmax=2, kmax=q.shape[-2])
-        qb2, qb2_pl = torch.empty_like(q), torch.empty_like(q_pl)
-        chb, chb_pl = torch.empty_like(ch), torch.empty_like(ch_pl)
-        nctx.horizontal_limiter_thuburn_adjoint(None, None, qb2, qb2_pl, pb, pb_pl, None, None, *fixed, chb, chb_pl)
-        return (None, qab, qab_pl, qb + qb2, qb_pl + qb2_pl, None, None, chb, chb_pl, None, None)
 
 
 def _c(g, ref):
@@ -158,46 +121,67 @@ class Courant(torch.autograd.Function):
         return None, fb, fb_pl, rb, rb_pl
 
 
-class Gradient(torch.autograd.Function):
-    """grad = the 7-point stencil of coef_grad on q (nicam_oprt_gradient)."""
+class FaceValues(torch.autograd.Function):
+    """One tracer's limited face values, as one node: the gradient (the 7-point
+    stencil of coef_grad, nicam_oprt_gradient), its halo exchange, the upwind
+    remap q + grad . (GRD_xc - GRD_x) (nicam_horizontal_remap) and the limiter in
+    the library's exchange mode (HLIM:42-430: the allowable range Qout_prev, its
+    halo exchange and the clamp, one masked call); cmask, d, coef_grad and GRD_x
+    held fixed.  The transpose runs the stages' adjoints in reverse: the faces'
+    half pass of the limiter's (q_a_b -> q_a's, q's and Qout_post's cotangents),
+    the exchange's, the rows' half pass (Qout_prev's -> q's and ch's), the
+    remap's, the exchange's and the gradient's.  A node per stage costs the host
+    more than the kernels cost the GPU on small grids (a gradient of two steps of
+    three tracers, 40 regions of 18x18 x 42: 6.5 ms with the vertical stages
+    apart too, 5.4 ms with one node each), and a copy of every array that a
+    stage updates in place."""
 
     @staticmethod
-    def forward(fctx, nctx: Context, cg, cg_pl, q, q_pl):
-        grad = q.new_empty((3,) + q.shape)
-        grad_pl = q_pl.new_empty((3,) + q_pl.shape)
+    def forward(fctx, nctx: Context, cg, cg_pl, X, X_pl, d, d_pl, cm, cm_pl, q, q_pl, xc, xc_pl, ch, ch_pl):
+        q, q_pl = q.contiguous(), q_pl.contiguous()
+        grad, grad_pl = q.new_empty((3,) + q.shape), q_pl.new_empty((3,) + q_pl.shape)
         nctx.oprt_gradient(grad, grad_pl, q, q_pl, cg, cg_pl)
-        fctx.nctx, fctx.cg, fctx.cg_pl = nctx, cg, cg_pl
-        return grad, grad_pl
-
-    @staticmethod
-    def backward(fctx, g, g_pl):
-        b, b_pl = g.new_empty(g.shape[1:]), g_pl.new_empty(g_pl.shape[1:])
-        fctx.nctx.oprt_gradient_adjoint(b, b_pl, _c(g, g), _c(g_pl, g_pl), fctx.cg, fctx.cg_pl)
-        return None, None, None, b, b_pl
-
-
-class Remap(torch.autograd.Function):
-    """Upwind face values q + grad . (GRD_xc - GRD_x) (nicam_horizontal_remap)
-    into zeroed arrays; cmask and GRD_x held fixed."""
-
-    @staticmethod
-    def forward(fctx, nctx: Context, cm, cm_pl, X, X_pl, q, q_pl, grad, grad_pl, xc, xc_pl):
-        q_a, q_a_pl = q.new_zeros((6,) + q.shape), q_pl.new_zeros(q_pl.shape)
-        nctx.horizontal_remap(q_a, q_a_pl, q, q_pl, grad, grad_pl, cm, cm_pl, xc, xc_pl, X, X_pl)
+        nctx.comm_data_transfer(grad, grad_pl, vmax=3, kmax=q.shape[-2])
+        out, out_pl = q.new_zeros((6,) + q.shape), q_pl.new_zeros(q_pl.shape)
+        nctx.horizontal_remap(out, out_pl, q, q_pl, grad, grad_pl, cm, cm_pl, xc, xc_pl, X, X_pl)
+        post, post_pl = q.new_empty((2,) + q.shape), q_pl.new_zeros((2,) + q_pl.shape)
+        mask = torch.empty(q.shape, dtype=torch.uint8, device=q.device)
+        mask_pl = torch.empty(q_pl.shape, dtype=torch.uint8, device=q.device)
+        nctx.horizontal_limiter_thuburn_mask(out, out_pl, q, q_pl, d, d_pl, ch, ch_pl, cm, cm_pl, post, post_pl,
+                                             None, None, mask, mask_pl)
         fctx.nctx = nctx
-        fctx.save_for_backward(grad, grad_pl, cm, cm_pl, xc, xc_pl, X, X_pl)
-        return q_a, q_a_pl
+        fctx.save_for_backward(cg, cg_pl, X, X_pl, d, d_pl, cm, cm_pl, q, q_pl, xc, xc_pl, ch, ch_pl, grad, grad_pl,
+                               out, out_pl, post, post_pl, mask, mask_pl)
+        return out, out_pl
 
     @staticmethod
     def backward(fctx, g, g_pl):
-        grad, grad_pl, cm, cm_pl, xc, xc_pl, X, X_pl = fctx.saved_tensors
-        qb, qb_pl = grad.new_empty(grad.shape[1:]), grad_pl.new_empty(grad_pl.shape[1:])
+        (cg, cg_pl, X, X_pl, d, d_pl, cm, cm_pl, q, q_pl, xc, xc_pl, ch, ch_pl, grad, grad_pl, out, out_pl, post,
+         post_pl, mask, mask_pl) = fctx.saved_tensors
+        nctx, kmax = fctx.nctx, q.shape[-2]
+        qab = torch.zeros_like(out) if g is None else g.contiguous().clone()
+        qab_pl = torch.zeros_like(out_pl) if g_pl is None else g_pl.contiguous().clone()
+        qb, qb_pl = torch.empty_like(q), torch.empty_like(q_pl)
+        part, part_pl = torch.empty_like(q), torch.empty_like(q_pl)  # q's cotangent through one stage
+        pb, pb_pl = torch.empty_like(post), torch.empty_like(post_pl)
+        chb, chb_pl = torch.empty_like(ch), torch.empty_like(ch_pl)
+        fixed = (out, out_pl, q, q_pl, d, d_pl, ch, ch_pl, cm, cm_pl, post, post_pl, mask, mask_pl)
+        nctx.horizontal_limiter_thuburn_adjoint(qab, qab_pl, qb, qb_pl, None, None, pb, pb_pl, *fixed)
+        nctx.comm_data_transfer_adjoint(pb, pb_pl, vmax=2, kmax=kmax)
+        nctx.horizontal_limiter_thuburn_adjoint(None, None, part, part_pl, pb, pb_pl, None, None, *fixed, chb, chb_pl)
+        qb.add_(part)
+        qb_pl.add_(part_pl)
         gb, gb_pl = torch.empty_like(grad), torch.empty_like(grad_pl)
         xb, xb_pl = torch.empty_like(xc), torch.empty_like(xc_pl)
-        g = qb.new_zeros((6,) + qb.shape) if g is None else g.contiguous()
-        fctx.nctx.horizontal_remap_adjoint(qb, qb_pl, gb, gb_pl, xb, xb_pl, g, _c(g_pl, qb_pl), grad, grad_pl, cm,
-                                           cm_pl, xc, xc_pl, X, X_pl)
-        return None, None, None, None, None, qb, qb_pl, gb, gb_pl, xb, xb_pl
+        nctx.horizontal_remap_adjoint(part, part_pl, gb, gb_pl, xb, xb_pl, qab, qab_pl, grad, grad_pl, cm, cm_pl, xc,
+                                      xc_pl, X, X_pl)
+        qb.add_(part)
+        qb_pl.add_(part_pl)
+        nctx.comm_data_transfer_adjoint(gb, gb_pl, vmax=3, kmax=kmax)
+        nctx.oprt_gradient_adjoint(part, part_pl, gb, gb_pl, cg, cg_pl)
+        qb.add_(part)
+        qb_pl.add_(part_pl)
+        return (None,) * 9 + (qb, qb_pl, xb, xb_pl, chb, chb_pl)
 
 
 class Update(torch.autograd.Function):
@@ -245,24 +229,45 @@ class VCourant(torch.autograd.Function):
         return None, fb, fb_pl, rb, rb_pl
 
 
-class VFace(torch.autograd.Function):
-    """q_h = afact q(k) + bfact q(k-1) on the interior half levels, 0 on the
-    others (nicam_vertical_face into a zeroed array), for one tracer."""
+class VerticalTransport(torch.autograd.Function):
+    """One tracer's vertical half, as one node: the half-level values q_h = afact
+    q(k) + bfact q(k-1) on the interior half levels, 0 on the others
+    (nicam_vertical_face), vertical_limiter_thuburn (VLIM:41-243, masked) and
+    rhogq less the flux divergence of flx_v * q_h on kmin..kmax
+    (nicam_tracer_update_vertical); d and the inflow flags held fixed."""
 
     @staticmethod
-    def forward(fctx, nctx: Context, q, q_pl):
+    def forward(fctx, nctx: Context, d, d_pl, q, q_pl, rq, rq_pl, flx_v, flx_v_pl, ck, ck_pl):
+        q, q_pl = q.contiguous(), q_pl.contiguous()
         q_h, q_h_pl = torch.zeros_like(q), torch.zeros_like(q_pl)
         nctx.vertical_face(q_h, q_h_pl, q, q_pl)
+        M, MP = nctx.vlim_mask_words()
+        mask = torch.empty(M, dtype=torch.int32, device=q.device)
+        mask_pl = torch.empty(max(MP, 1), dtype=torch.int32, device=q.device)[:MP]
+        nctx.vertical_limiter_thuburn_mask(q_h, q_h_pl, q, q_pl, d, d_pl, ck, ck_pl, mask, mask_pl)
+        out, out_pl = rq.contiguous().clone(), rq_pl.contiguous().clone()
+        nctx.tracer_update_vertical(out, out_pl, flx_v, flx_v_pl, q_h, q_h_pl)
         fctx.nctx = nctx
-        fctx.save_for_backward(q, q_pl)
-        return q_h, q_h_pl
+        fctx.save_for_backward(d, d_pl, q, q_pl, flx_v, flx_v_pl, ck, ck_pl, q_h, q_h_pl, mask, mask_pl)
+        return out, out_pl
 
     @staticmethod
     def backward(fctx, g, g_pl):
-        q, q_pl = fctx.saved_tensors
+        d, d_pl, q, q_pl, flx_v, flx_v_pl, ck, ck_pl, q_h, q_h_pl, mask, mask_pl = fctx.saved_tensors
+        nctx = fctx.nctx
+        g, g_pl = _c(g, flx_v), _c(g_pl, flx_v_pl)
+        fb, fb_pl = torch.empty_like(flx_v), torch.empty_like(flx_v_pl)
+        qhb, qhb_pl = torch.empty_like(q_h), torch.empty_like(q_h_pl)
+        nctx.tracer_update_vertical_adjoint(fb, fb_pl, qhb, qhb_pl, g, g_pl, flx_v, flx_v_pl, q_h, q_h_pl)
         qb, qb_pl = torch.empty_like(q), torch.empty_like(q_pl)
-        fctx.nctx.vertical_face_adjoint(qb, qb_pl, _c(g, q), _c(g_pl, q_pl))
-        return None, qb, qb_pl
+        ckb, ckb_pl = torch.empty_like(ck), torch.empty_like(ck_pl)
+        nctx.vertical_limiter_thuburn_adjoint(qhb, qhb_pl, qb, qb_pl, q_h, q_h_pl, q, q_pl, d, d_pl, ck, ck_pl, mask,
+                                              mask_pl, ckb, ckb_pl)
+        part, part_pl = torch.empty_like(q), torch.empty_like(q_pl)
+        nctx.vertical_face_adjoint(part, part_pl, qhb, qhb_pl)
+        qb.add_(part)
+        qb_pl.add_(part_pl)
+        return None, None, None, qb, qb_pl, g, g_pl, fb, fb_pl, ckb, ckb_pl
 
 
 class VUpdate(torch.autograd.Function):
@@ -325,6 +330,9 @@ class TracerStep:
         self.vi = {k + s: T(vi[k + s]) for k in VI_IN for s in ("", "_pl")}
         self.rhogw_in, self.rhogw_in_pl = T(vi["rhogw"]), T(vi["rhogw_pl"])
         self.rdgz = T(fac["rdgz"])
+        # the face values of the density's own update, held by every step's graph
+        self.ones = torch.ones((6,) + self.rhogw_in.shape, dtype=torch.float64, device=dev)
+        self.ones_pl = torch.ones_like(self.rhogw_in_pl)
         inner = np.zeros((n1, n1), dtype=bool)
         inner[1:-1, 1:-1] = True
         self.inner = torch.from_numpy(inner.reshape(-1)).to(dev)
@@ -351,17 +359,6 @@ class TracerStep:
     def courant(self, flx, flx_pl, rhog, rhog_pl):
         return Courant.apply(self.ctx, flx, flx_pl, rhog, rhog_pl)
 
-    def gradient(self, q, q_pl):
-        """q [l][k][g] -> grad [3][l][k][g] on the flat range gmin..gmax (zero
-        elsewhere); the pole centre from its ring."""
-        return Gradient.apply(self.ctx, self.cg, self.cg_pl, q.contiguous(), q_pl.contiguous())
-
-    def remap(self, q, q_pl, grad, grad_pl, cm, cm_pl, xc, xc_pl):
-        """Upwind face values q + grad.(GRD_xc - GRD_x) of every arc from the
-        origins i, j in [gmin-1, gmax]; the faces no arc reaches stay 0."""
-        return Remap.apply(self.ctx, cm, cm_pl, self.X, self.X_pl, q.contiguous(), q_pl.contiguous(),
-                           grad.contiguous(), grad_pl.contiguous(), xc, xc_pl)
-
     def hupdate(self, rq, rq_pl, flx, flx_pl, q_a, q_a_pl):
         """rq [l][k][g] (one tracer) less the sum of flx * q_a over the faces."""
         return Update.apply(self.ctx, rq, rq_pl, flx, flx_pl, q_a.contiguous(), q_a_pl.contiguous())
@@ -373,14 +370,12 @@ class TracerStep:
         ck, ck_pl = VCourant.apply(ctx, flx_v, flx_v_pl, rhog, rhog_pl)
         ck, ck_pl = ck.contiguous(), ck_pl.contiguous()
         outs, outs_pl = [], []
-        for t in range(q.shape[0]):
-            qt, qt_pl = q[t].contiguous(), q_pl[t].contiguous()
-            q_h, q_h_pl = VFace.apply(ctx, qt, qt_pl)
-            a, b = VerticalLimiter.apply(ctx, q_h, q_h_pl, qt, qt_pl, self.dv, self.dv_pl, ck, ck_pl)
-            a, b = VUpdate.apply(ctx, rq[t], rq_pl[t], flx_v, flx_v_pl, a.contiguous(), b.contiguous())
+        # unbind, not q[t]: an index's transpose is a zeroed copy of every tracer, added up per tracer
+        for qt, qt_pl, rqt, rqt_pl in zip(q.unbind(0), q_pl.unbind(0), rq.unbind(0), rq_pl.unbind(0)):
+            a, b = VerticalTransport.apply(ctx, self.dv, self.dv_pl, qt, qt_pl, rqt, rqt_pl, flx_v, flx_v_pl, ck, ck_pl)
             outs.append(a)
             outs_pl.append(b)
-        ones, ones_pl = torch.ones_like(rhog), torch.ones_like(rhog_pl)
+        ones, ones_pl = self.ones[0], self.ones_pl
         rhog, rhog_pl = VUpdate.apply(ctx, rhog, rhog_pl, flx_v, flx_v_pl, ones, ones_pl)
         return torch.stack(outs), torch.stack(outs_pl), rhog, rhog_pl
 
@@ -388,12 +383,8 @@ class TracerStep:
     def face_values(self, q, q_pl, xc, xc_pl, cm, cm_pl, ch, ch_pl):
         """One tracer's limited face values: gradient, exchange, remap, the
         limiter's allowable range, its exchange, the clamp."""
-        ctx = self.ctx
-        grad, grad_pl = self.gradient(q, q_pl)
-        grad, grad_pl = self.halo(grad, grad_pl)
-        q_a, q_a_pl = self.remap(q, q_pl, grad, grad_pl, cm, cm_pl, xc, xc_pl)
-        q, q_pl, q_a, q_a_pl = q.contiguous(), q_pl.contiguous(), q_a.contiguous(), q_a_pl.contiguous()
-        return HorizontalLimiter.apply(ctx, q_a, q_a_pl, q, q_pl, self.d, self.d_pl, ch, ch_pl, cm, cm_pl)
+        return FaceValues.apply(self.ctx, self.cg, self.cg_pl, self.X, self.X_pl, self.d, self.d_pl, cm, cm_pl, q, q_pl,
+                                xc, xc_pl, ch, ch_pl)
 
     def __call__(self, q, q_pl, rhog, rhog_pl, recompute_tracers: bool = False):
         """One step.  recompute_tracers: each tracer's face values are
@@ -406,18 +397,19 @@ class TracerStep:
         flx, flx_pl, xc, xc_pl = HorizontalFlux.apply(ctx, self.dt, rhog, rhog_pl, *self.rv)
         ch, ch_pl, cm, cm_pl = self.courant(flx, flx_pl, rhog, rhog_pl)
         ch, ch_pl = ch.contiguous(), ch_pl.contiguous()
+        qs, qs_pl = q.unbind(0), q_pl.unbind(0)
         qas, qas_pl = [], []
         for t in range(ntr):
-            args = (q[t], q_pl[t], xc, xc_pl, cm, cm_pl, ch, ch_pl)
+            args = (qs[t], qs_pl[t], xc, xc_pl, cm, cm_pl, ch, ch_pl)
             if recompute_tracers:
                 q_a, q_a_pl = checkpoint(self.face_values, *args, use_reentrant=False)
             else:
                 q_a, q_a_pl = self.face_values(*args)
             qas.append(q_a)
             qas_pl.append(q_a_pl)
-        rqs = [self.hupdate(rhog * q[t], rhog_pl * q_pl[t], flx, flx_pl, qas[t], qas_pl[t]) for t in range(ntr)]
+        rqs = [self.hupdate(rhog * qs[t], rhog_pl * qs_pl[t], flx, flx_pl, qas[t], qas_pl[t]) for t in range(ntr)]
         rq, rq_pl = torch.stack([a for a, _ in rqs]), torch.stack([b for _, b in rqs])
-        ones, ones_pl = torch.ones_like(flx), torch.ones_like(flx_pl)
+        ones, ones_pl = self.ones, self.ones_pl
         rhog1, rhog1_pl = self.hupdate(rhog, rhog_pl, flx, flx_pl, ones, ones_pl)
         q1, q1_pl = rq / rhog1, rq_pl / rhog1_pl
         # vertical: rho*w from the solve on the step's density, its flux fixed to a multiple of it
