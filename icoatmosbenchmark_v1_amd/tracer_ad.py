@@ -72,6 +72,44 @@ class HorizontalFlux(torch.autograd.Function):
         return (None, None, *b)
 
 
+class HorizontalLimiter(torch.autograd.Function):
+    """q_a' = horizontal_limiter_thuburn(q_a, q, ch; d, cmask) (HLIM:42-430) in
+    the library's exchange mode: the allowable range Qout_prev, its halo
+    exchange (Qout_post) and the clamp, one masked call; d and cmask held fixed.
+    Its transpose: the faces' half pass of the limiter's adjoint (q_a_b ->
+    q_a's, q's and Qout_post's cotangents), the halo exchange's transpose
+    (Qout_post's -> Qout_prev's) and the rows' half pass (Qout_prev's -> q's and
+    ch's)."""
+
+    @staticmethod
+    def forward(fctx, nctx: Context, q_a, q_a_pl, q, q_pl, d, d_pl, ch, ch_pl, cm, cm_pl):
+        out, out_pl = q_a.clone(), q_a_pl.clone()
+        post, post_pl = q.new_empty((2,) + q.shape), q_pl.new_zeros((2,) + q_pl.shape)
+        mask = torch.empty(q.shape, dtype=torch.uint8, device=q.device)
+        mask_pl = torch.empty(q_pl.shape, dtype=torch.uint8, device=q.device)
+        nctx.horizontal_limiter_thuburn_mask(out, out_pl, q, q_pl, d, d_pl, ch, ch_pl, cm, cm_pl, post, post_pl,
+                                             None, None, mask, mask_pl)
+        fctx.nctx = nctx
+        fctx.save_for_backward(out, out_pl, q, q_pl, post, post_pl, d, d_pl, ch, ch_pl, cm, cm_pl, mask, mask_pl)
+        return out, out_pl
+
+    @staticmethod
+    def backward(fctx, g_qa, g_qa_pl):
+        out, out_pl, q, q_pl, post, post_pl, d, d_pl, ch, ch_pl, cm, cm_pl, mask, mask_pl = fctx.saved_tensors
+        nctx = fctx.nctx
+        qab = torch.zeros_like(out) if g_qa is None else g_qa.contiguous().clone()
+        qab_pl = torch.zeros_like(out_pl) if g_qa_pl is None else g_qa_pl.contiguous().clone()
+        qb, qb_pl = torch.empty_like(q), torch.empty_like(q_pl)
+        pb, pb_pl = torch.empty_like(post), torch.empty_like(post_pl)
+        fixed = (out, out_pl, q, q_pl, d, d_pl, ch, ch_pl, cm, cm_pl, post, post_pl, mask, mask_pl)
+        nctx.horizontal_limiter_thuburn_adjoint(qab, qab_pl, qb, qb_pl, None, None, pb, pb_pl, *fixed)
+        nctx.comm_data_transfer_adjoint(pb, pb_pl, vmax=2, kmax=q.shape[-2])
+        qb2, qb2_pl = torch.empty_like(q), torch.empty_like(q_pl)
+        chb, chb_pl = torch.empty_like(ch), torch.empty_like(ch_pl)
+        nctx.horizontal_limiter_thuburn_adjoint(None, None, qb2, qb2_pl, pb, pb_pl, None, None, *fixed, chb, chb_pl)
+        return (None, qab, qab_pl, qb + qb2, qb_pl + qb2_pl, None, None, chb, chb_pl, None, None)
+
+
 def _c(g, ref):
     """A cotangent autograd may give as None, as a contiguous tensor."""
     return torch.zeros_like(ref) if g is None else g.contiguous()
@@ -119,6 +157,48 @@ class Courant(torch.autograd.Function):
         fctx.nctx.tracer_courant_adjoint(fb, fb_pl, rb, rb_pl, _c(g_ch, flx), _c(g_ch_pl, flx_pl), flx, flx_pl, rhog,
                                          rhog_pl)
         return None, fb, fb_pl, rb, rb_pl
+
+
+class Gradient(torch.autograd.Function):
+    """grad = the 7-point stencil of coef_grad on q (nicam_oprt_gradient)."""
+
+    @staticmethod
+    def forward(fctx, nctx: Context, cg, cg_pl, q, q_pl):
+        grad = q.new_empty((3,) + q.shape)
+        grad_pl = q_pl.new_empty((3,) + q_pl.shape)
+        nctx.oprt_gradient(grad, grad_pl, q, q_pl, cg, cg_pl)
+        fctx.nctx, fctx.cg, fctx.cg_pl = nctx, cg, cg_pl
+        return grad, grad_pl
+
+    @staticmethod
+    def backward(fctx, g, g_pl):
+        b, b_pl = g.new_empty(g.shape[1:]), g_pl.new_empty(g_pl.shape[1:])
+        fctx.nctx.oprt_gradient_adjoint(b, b_pl, _c(g, g), _c(g_pl, g_pl), fctx.cg, fctx.cg_pl)
+        return None, None, None, b, b_pl
+
+
+class Remap(torch.autograd.Function):
+    """Upwind face values q + grad . (GRD_xc - GRD_x) (nicam_horizontal_remap)
+    into zeroed arrays; cmask and GRD_x held fixed."""
+
+    @staticmethod
+    def forward(fctx, nctx: Context, cm, cm_pl, X, X_pl, q, q_pl, grad, grad_pl, xc, xc_pl):
+        q_a, q_a_pl = q.new_zeros((6,) + q.shape), q_pl.new_zeros(q_pl.shape)
+        nctx.horizontal_remap(q_a, q_a_pl, q, q_pl, grad, grad_pl, cm, cm_pl, xc, xc_pl, X, X_pl)
+        fctx.nctx = nctx
+        fctx.save_for_backward(grad, grad_pl, cm, cm_pl, xc, xc_pl, X, X_pl)
+        return q_a, q_a_pl
+
+    @staticmethod
+    def backward(fctx, g, g_pl):
+        grad, grad_pl, cm, cm_pl, xc, xc_pl, X, X_pl = fctx.saved_tensors
+        qb, qb_pl = grad.new_empty(grad.shape[1:]), grad_pl.new_empty(grad_pl.shape[1:])
+        gb, gb_pl = torch.empty_like(grad), torch.empty_like(grad_pl)
+        xb, xb_pl = torch.empty_like(xc), torch.empty_like(xc_pl)
+        g = qb.new_zeros((6,) + qb.shape) if g is None else g.contiguous()
+        fctx.nctx.horizontal_remap_adjoint(qb, qb_pl, gb, gb_pl, xb, xb_pl, g, _c(g_pl, qb_pl), grad, grad_pl, cm,
+                                           cm_pl, xc, xc_pl, X, X_pl)
+        return None, None, None, None, None, qb, qb_pl, gb, gb_pl, xb, xb_pl
 
 
 class FaceValues(torch.autograd.Function):
@@ -227,6 +307,26 @@ class VCourant(torch.autograd.Function):
         g_pl = flx_v_pl.new_zeros((2,) + flx_v_pl.shape) if g_pl is None else g_pl.contiguous()
         fctx.nctx.vertical_courant_adjoint(fb, fb_pl, rb, rb_pl, g, g_pl, flx_v, flx_v_pl, rhog, rhog_pl)
         return None, fb, fb_pl, rb, rb_pl
+
+
+class VFace(torch.autograd.Function):
+    """q_h = afact q(k) + bfact q(k-1) on the interior half levels, 0 on the
+    others (nicam_vertical_face into a zeroed array), for one tracer."""
+
+    @staticmethod
+    def forward(fctx, nctx: Context, q, q_pl):
+        q_h, q_h_pl = torch.zeros_like(q), torch.zeros_like(q_pl)
+        nctx.vertical_face(q_h, q_h_pl, q, q_pl)
+        fctx.nctx = nctx
+        fctx.save_for_backward(q, q_pl)
+        return q_h, q_h_pl
+
+    @staticmethod
+    def backward(fctx, g, g_pl):
+        q, q_pl = fctx.saved_tensors
+        qb, qb_pl = torch.empty_like(q), torch.empty_like(q_pl)
+        fctx.nctx.vertical_face_adjoint(qb, qb_pl, _c(g, q), _c(g_pl, q_pl))
+        return None, qb, qb_pl
 
 
 class VerticalTransport(torch.autograd.Function):
@@ -358,6 +458,17 @@ class TracerStep:
 
     def courant(self, flx, flx_pl, rhog, rhog_pl):
         return Courant.apply(self.ctx, flx, flx_pl, rhog, rhog_pl)
+
+    def gradient(self, q, q_pl):
+        """q [l][k][g] -> grad [3][l][k][g] on the flat range gmin..gmax (zero
+        elsewhere); the pole centre from its ring."""
+        return Gradient.apply(self.ctx, self.cg, self.cg_pl, q.contiguous(), q_pl.contiguous())
+
+    def remap(self, q, q_pl, grad, grad_pl, cm, cm_pl, xc, xc_pl):
+        """Upwind face values q + grad.(GRD_xc - GRD_x) of every arc from the
+        origins i, j in [gmin-1, gmax]; the faces no arc reaches stay 0."""
+        return Remap.apply(self.ctx, cm, cm_pl, self.X, self.X_pl, q.contiguous(), q_pl.contiguous(),
+                           grad.contiguous(), grad_pl.contiguous(), xc, xc_pl)
 
     def hupdate(self, rq, rq_pl, flx, flx_pl, q_a, q_a_pl):
         """rq [l][k][g] (one tracer) less the sum of flx * q_a over the faces."""
