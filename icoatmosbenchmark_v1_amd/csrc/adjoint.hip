@@ -579,7 +579,8 @@ __global__ void __launch_bounds__(BLOCK_VLA) __attribute__((amdgpu_waves_per_eu(
 // work-item only.
 constexpr int HSW = 256;
 constexpr int HMAXI = 160;
-constexpr int HPOLE = 256;
+constexpr int HPOLE = 64;
+constexpr int kMaxGallPl = 15;  // nicam_ctx_create's bound on gall_pl
 
 struct HaArgs {
     double *qab, *qb, *Qpostb;
@@ -644,8 +645,6 @@ __host__ __device__ constexpr int arc_slot(int m, int d)
 }
 // ... of the singular-point arc (m = 1, origin 0): {0, iall+1, iall+2, iall}
 __host__ __device__ constexpr int arc_slot_sgp(int d) { return d == 4 ? 0 : d == 1 ? 1 : d == 0 ? 2 : d == 2 ? 3 : -1; }
-
-__global__ void __launch_bounds__(HPOLE) hlim_adjoint_pole(HaArgs A);
 
 // four waves per SIMD (the LDS ring allows four work-groups per CU): 1.57 ms at gl7, against 1.87 ms at
 // three and 2.25 ms at two, despite the registers the cap spills
@@ -986,44 +985,61 @@ __global__ void __launch_bounds__(HSW) __attribute__((amdgpu_waves_per_eu(CHB ? 
 }
 
 // Poles: one work-item per (k, l) slab, sequential as the oracle (HLIM:307-363,
-// 412-425); it owns the slab's pole arrays, so no atomics.
+// 412-425); it owns the slab's pole arrays, so no atomics.  NPL: gall_pl where it
+// is known at compile time (6, the ring every NICAM grid has): the ring's inputs
+// load at once and its sums stay in registers, where a walk through memory paid
+// a round trip per term (24 us at 98 levels, behind the regions' kernel; now
+// 10.5 us).  0: any size.
+template <int NPL>
 __global__ void __launch_bounds__(HPOLE) hlim_adjoint_pole(HaArgs A)
 {
     const int t = blockIdx.x * HPOLE + threadIdx.x;
-    const int kall = A.kall, npl = A.gall_pl;
+    const int kall = A.kall, npl = NPL > 0 ? NPL : A.gall_pl;
+    constexpr int N = NPL > 0 ? NPL : kMaxGallPl, U = NPL > 0 ? NPL : 1;
     if (!A.have_pl || t >= kall * kLallPl) return;
     const int k = t % kall, l = t / kall;
     const size_t fb = ((size_t)l * kall + k) * npl;
     const size_t pplane = (size_t)kLallPl * kall * npl;
-    const double *qs = A.q_pl + fb, *chs = A.ch_pl + fb, *cms = A.cmask_pl + fb;
-    // the rows run when Qout_prev_b is given, the faces when q_a_b is
-    double *xq = A.qb_pl + fb, *xa = A.qab_pl ? A.qab_pl + fb : nullptr, *xp = A.Qpostb_pl ? A.Qpostb_pl + fb : nullptr;
-    for (int v = 0; v < npl; ++v) {
-        xq[v] = 0.0;
-        if (xp) {
-            xp[v] = 0.0;
-            xp[pplane + v] = 0.0;
-        }
+    double qs[N], chs[N], cms[N];
+#pragma unroll U
+    for (int v = 0; v < N; ++v) {
+        const int u = v < npl ? v : 0;
+        qs[v] = A.q_pl[fb + u];
+        chs[v] = A.ch_pl[fb + u];
+        cms[v] = A.cmask_pl[fb + u];
     }
+    // the rows run when Qout_prev_b is given, the faces when q_a_b is
+    double *xa = A.qab_pl ? A.qab_pl + fb : nullptr;
+    double xq[N], xp0[N], xp1[N];  // the cotangents of q and of Qout_post's two bounds
+#pragma unroll U
+    for (int v = 0; v < N; ++v) xq[v] = xp0[v] = xp1[v] = 0.0;
+    // x[i] += y where the index is known at run time only
+    auto add = [&](double (&x)[N], int i, double y) {
+#pragma unroll U
+        for (int v = 0; v < N; ++v) x[v] = v == i ? x[v] + y : x[v];
+    };
     const double BIG = A.big;
     auto arc = [&](int v, int &il, int &ih, double &lo_v, double &hi_v) {
         int vp1 = v + 1, vm1 = v - 1;
         if (vp1 == npl) vp1 = 1;
         if (vm1 == 0) vm1 = npl - 1;
-        const int c4[4] = {0, v, vm1, vp1};
         lo_v = qs[0];
         hi_v = lo_v;
         il = 0;
         ih = 0;
-        for (int u = 1; u < 4; ++u) {
-            const double x = qs[c4[u]];
-            if (x < lo_v) { lo_v = x; il = c4[u]; }
-            if (x > hi_v) { hi_v = x; ih = c4[u]; }
-        }
+        auto see = [&](int c) {
+            const double x = qs[c];
+            if (x < lo_v) { lo_v = x; il = c; }
+            if (x > hi_v) { hi_v = x; ih = c; }
+        };
+        see(v);
+        see(vm1);
+        see(vp1);
     };
     const double qn = qs[0];
     int smin = -1, smax = -1;
     double nmin = qn, nmax = qn;
+#pragma unroll U
     for (int v = 1; v < npl; ++v) {
         int il, ih;
         double lv, hv;
@@ -1034,6 +1050,7 @@ __global__ void __launch_bounds__(HPOLE) hlim_adjoint_pole(HaArgs A)
         if (mx1 > nmax) { nmax = mx1; smax = v; }
     }
     double Cin = 0.0, Cout = 0.0;
+#pragma unroll U
     for (int v = 1; v < npl; ++v) {
         const double chm = cms[v] * chs[v];
         Cin = Cin + chm;
@@ -1045,6 +1062,7 @@ __global__ void __launch_bounds__(HPOLE) hlim_adjoint_pole(HaArgs A)
     if (A.chb_pl) {
         // Qout in ch(v): cmask*ch enters Cin and CQin, ch - cmask*ch Cout
         double CQmin = 0.0, CQmax = 0.0;
+#pragma unroll U
         for (int v = 1; v < npl; ++v) {
             int il, ih;
             double lv, hv;
@@ -1058,6 +1076,7 @@ __global__ void __launch_bounds__(HPOLE) hlim_adjoint_pole(HaArgs A)
         const double b0 = A.Qprevb_pl[fb], b1 = A.Qprevb_pl[pplane + fb];
         double *xc = A.chb_pl + fb;
         xc[0] = 0.0;
+#pragma unroll U
         for (int v = 1; v < npl; ++v) {
             int il, ih;
             double lv, hv;
@@ -1069,27 +1088,37 @@ __global__ void __launch_bounds__(HPOLE) hlim_adjoint_pole(HaArgs A)
             xc[v] = (b0 != 0.0 ? b0 * d0 : 0.0) + (b1 != 0.0 ? b1 * d1 : 0.0);
         }
     }
-    for (int mm = 0; mm < 2 && A.Qprevb_pl; ++mm) {
+#pragma unroll U
+    for (int mm = 0; mm < 2; ++mm) {
+        if (!A.Qprevb_pl) break;
         const double bq = A.Qprevb_pl[(size_t)mm * pplane + fb];
         const int sel = mm == 0 ? smax : smin;
         xq[0] = xq[0] + (fac + zerosw) * bq;
         int selc = 0;
-        if (sel >= 0) {
+        double selm = 1.0;
+#pragma unroll U
+        for (int v = 1; v < npl; ++v) {
             int il, ih;
             double lv, hv;
-            arc(sel, il, ih, lv, hv);
-            selc = mm == 0 ? ih : il;
+            arc(v, il, ih, lv, hv);
+            if (v == sel) {
+                selc = mm == 0 ? ih : il;
+                selm = cms[v];
+            }
         }
-        xq[selc] = xq[selc] + (-(fac * E) * (sel < 0 ? 1.0 : cms[sel])) * bq;
+        add(xq, selc, (-(fac * E) * selm) * bq);
+#pragma unroll U
         for (int v = 1; v < npl; ++v) {
             int il, ih;
             double lv, hv;
             arc(v, il, ih, lv, hv);
             const int cx = mm == 0 ? ih : il;
-            xq[cx] = xq[cx] + (-(fac * (cms[v] * chs[v])) * cms[v]) * bq;
+            add(xq, cx, (-(fac * (cms[v] * chs[v])) * cms[v]) * bq);
         }
     }
-    for (int v = 1; v < npl && xa; ++v) {
+#pragma unroll U
+    for (int v = 1; v < npl; ++v) {
+        if (!xa) break;
         const double c = cms[v];
         const int T = c > 0.0 ? v : 0;
         int kind = 0, cell = 0;
@@ -1105,9 +1134,17 @@ __global__ void __launch_bounds__(HPOLE) hlim_adjoint_pole(HaArgs A)
         }
         const double ob = xa[v];
         xa[v] = kind == 0 ? ob : 0.0;
-        if (kind == 1) xp[T] = xp[T] + ob;
-        else if (kind == 2) xp[pplane + T] = xp[pplane + T] + ob;
-        else if (kind >= 3) xq[cell] = xq[cell] + ob;
+        if (kind == 1) add(xp0, T, ob);
+        else if (kind == 2) add(xp1, T, ob);
+        else if (kind >= 3) add(xq, cell, ob);
+    }
+#pragma unroll U
+    for (int v = 0; v < npl; ++v) {
+        A.qb_pl[fb + v] = xq[v];
+        if (A.Qpostb_pl) {
+            A.Qpostb_pl[fb + v] = xp0[v];
+            A.Qpostb_pl[pplane + fb + v] = xp1[v];
+        }
     }
 }
 
@@ -1386,26 +1423,33 @@ __global__ void __launch_bounds__(FSW) __attribute__((amdgpu_waves_per_eu(2, 8))
 }
 
 // Poles: one work-item per (k, l), in the oracle's order (FLX:326-374).
+// NPL as hlim_adjoint_pole's (22 us at 98 levels, its arrays in scratch memory; now
+// 6.2 us).
+template <int NPL>
 __global__ void hflux_adjoint_pole(FaArgs A)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    const int kall = A.kall, npl = A.gall_pl;
-    if (!A.have_pl || t >= kall * kLallPl || npl > 16) return;
+    const int kall = A.kall, npl = NPL > 0 ? NPL : A.gall_pl;
+    constexpr int N = NPL > 0 ? NPL : kMaxGallPl, U = NPL > 0 ? NPL : 1;
+    if (!A.have_pl || t >= kall * kLallPl) return;
     const int k = t % kall, l = t / kall;
     const size_t fb = ((size_t)l * kall + k) * npl;
     const size_t pplane = (size_t)kLallPl * kall * npl, mstr = (size_t)kLallPl * npl, mb = (size_t)l * npl;
     const double dt = A.dt, EPS = A.eps;
     auto PT = [&](int v, int w) { return A.gt_pl[(size_t)w * mstr + mb + v]; };  // w: 2,3,4 = W1..W3
     const double ran = A.gp_pl[1 * mstr + mb + 0] * dt;
-    double Tv[4][16], Tb[4][16];
+    double Tv[4][N], Tb[4][N];
+#pragma unroll U
     for (int v = 1; v < npl; ++v) {
         const int vp1 = (v + 1 == npl) ? 1 : v + 1;
+#pragma unroll U
         for (int f = 0; f < 4; ++f) {
             const double *x = A.X_pl[f] + fb;
             Tv[f][v] = x[0] * PT(v, 2) + x[v] * PT(v, 3) + x[vp1] * PT(v, 4);
             Tb[f][v] = 0.0;
         }
     }
+#pragma unroll U
     for (int v = 1; v < npl; ++v) {
         const int vm1 = (v == 1) ? npl - 1 : v - 1;
         double s2[4];
@@ -1426,15 +1470,20 @@ __global__ void hflux_adjoint_pole(FaArgs A)
             Tb[f][v] += bv[f];
         }
     }
+#pragma unroll U
     for (int f = 0; f < 4; ++f) {
-        double *y = A.Xb_pl[f] + fb;
-        for (int v = 0; v < npl; ++v) y[v] = 0.0;
+        double y[N];
+#pragma unroll U
+        for (int v = 0; v < N; ++v) y[v] = 0.0;
+#pragma unroll U
         for (int v = 1; v < npl; ++v) {
             const int vp1 = (v + 1 == npl) ? 1 : v + 1;
             y[0] += Tb[f][v] * PT(v, 2);
             y[v] += Tb[f][v] * PT(v, 3);
             y[vp1] += Tb[f][v] * PT(v, 4);
         }
+#pragma unroll U
+        for (int v = 0; v < npl; ++v) A.Xb_pl[f][fb + v] = y[v];
     }
 }
 
@@ -1446,7 +1495,7 @@ int launch_hflux_adjoint(nicam_ctx c, const double *flxb, const double *flxb_pl,
 {
     const Dims &D = c->d;
     if (D.gall_1d > 160) return fail(NICAM_ERR_ARG, "gall_1d larger than the LDS tiles (160)");
-    if (D.have_pl && D.gall_pl > 16) return fail(NICAM_ERR_ARG, "gall_pl larger than 16");
+    if (D.have_pl && D.gall_pl > kMaxGallPl) return fail(NICAM_ERR_ARG, "gall_pl larger than 15");
     FaArgs A;
     A.flxb = flxb; A.xcb = xcb; A.flxb_pl = flxb_pl; A.xcb_pl = xcb_pl;
     for (int f = 0; f < 4; ++f) {
@@ -1478,8 +1527,8 @@ int launch_hflux_adjoint(nicam_ctx c, const double *flxb, const double *flxb_pl,
     else rc = launch(hflux_adjoint_kernel<FSW + 2 * 160 + 1>, FSW + 2 * 160 + 1);
     if (rc != NICAM_OK) return rc;
     if (D.have_pl)
-        hipLaunchKernelGGL(hflux_adjoint_pole, dim3((unsigned)((D.kall * kLallPl + 63) / 64)), dim3(64), 0, c->stream,
-                           A);
+        hipLaunchKernelGGL(D.gall_pl == 6 ? hflux_adjoint_pole<6> : hflux_adjoint_pole<0>,
+                           dim3((unsigned)((D.kall * kLallPl + 63) / 64)), dim3(64), 0, c->stream, A);
     NICAM_HIP(hipGetLastError());
     return NICAM_OK;
 }
@@ -1529,8 +1578,8 @@ int launch_hlim_adjoint(nicam_ctx c, double *qab, double *qab_pl, double *qb, do
     else
         hipLaunchKernelGGL((hlim_adjoint_kernel<false, 2>), dim3((unsigned)nslab), dim3(HSW), lds, c->stream, A);
     if (D.have_pl)
-        hipLaunchKernelGGL(hlim_adjoint_pole, dim3((unsigned)((D.kall * kLallPl + HPOLE - 1) / HPOLE)), dim3(HPOLE),
-                           0, c->stream, A);
+        hipLaunchKernelGGL(D.gall_pl == 6 ? hlim_adjoint_pole<6> : hlim_adjoint_pole<0>,
+                           dim3((unsigned)((D.kall * kLallPl + HPOLE - 1) / HPOLE)), dim3(HPOLE), 0, c->stream, A);
     NICAM_HIP(hipGetLastError());
     return NICAM_OK;
 }
