@@ -122,6 +122,7 @@ __global__ void __launch_bounds__(BLK) courant_kernel(CourantArgs A)
 constexpr int RCH = 256;   // output cells per remap work-group
 constexpr int RMAXI = 160; // largest gall_1d the remap tiles hold
 constexpr int RNO = 2;     // arc origins per work-item: RCH*RNO >= RCH + RMAXI + 1
+static_assert(3 * RCH >= RCH + 2 * RMAXI + 2, "remap_kernel<3> covers the widest region");
 
 struct RemapArgs {
     double *q_a, *q_a_pl;
@@ -161,7 +162,12 @@ __device__ void remap_pole(const RemapArgs &A, long p)
 // and qn from the far end, into LDS, and (phase 2) every cell picks each of
 // its six faces by that face's own mask: faces 1-3 from its own arcs, faces
 // 4-6 from the arcs of im1j (AI), im1jm1 (AIJ) and ijm1 (AJ).  A face no arc
-// reaches keeps its value.
+// reaches keeps its value.  The next level's inputs are loaded into registers
+// while phase 2 stores this one's faces (34x34x78x40 198 us with the loads
+// waited for at the head of each level and three barriers, 166 now; 66x66x98x40
+// 872 -> 753).  NSTG: staged cells per
+// work-item, NSTG * RCH >= RCH + 2 * gall_1d + 2.
+template <int NSTG>
 __global__ void __launch_bounds__(RCH) remap_kernel(RemapArgs A)
 {
     extern __shared__ double lds[];
@@ -206,23 +212,40 @@ __global__ void __launch_bounds__(RCH) remap_kernel(RemapArgs A)
     const bool f4 = active && i >= 1 && j <= last, f5 = active && i >= 1 && j >= 1,
                f6 = active && i <= last && j >= 1;
 
-    for (int k = k0; k < k1; ++k) {
+    double xcv[RNO][9], cm[6], stg[NSTG][4];
+    auto load_arcs = [&](int k) {  // my origins' arc centroids; q and its gradient of my staged cells
         const size_t fb = ((size_t)l * kall + k) * gall;
-        // loads that do not wait for the tile: my origins' arc centroids and my faces' masks
-        double xcv[RNO][9];
 #pragma unroll
         for (int r = 0; r < RNO; ++r)
 #pragma unroll
             for (int m = 0; m < 9; ++m) xcv[r][m] = org[r] >= 0 ? A.xc[(size_t)m * plane + fb + org[r]] : 0.0;
-        double cm[6];
+#pragma unroll
+        for (int u = 0; u < NSTG; ++u) {
+            const int s = tid + u * RCH, p = lo + s;
+            const bool ok = s < n_in && p >= 0 && p < gall;
+            stg[u][0] = ok ? A.q[fb + p] : 0.0;
+#pragma unroll
+            for (int d = 0; d < 3; ++d) stg[u][1 + d] = ok ? A.grad[d * plane + fb + p] : 0.0;
+        }
+    };
+    auto load_masks = [&](int k) {
+        const size_t fb = ((size_t)l * kall + k) * gall;
 #pragma unroll
         for (int f = 0; f < 6; ++f) cm[f] = active ? A.cmask[(size_t)f * plane + fb + g] : 0.0;
-        for (int s = tid; s < n_in; s += RCH) {
-            const int p = lo + s;
-            const bool ok = p >= 0 && p < gall;
-            s_q[s] = ok ? A.q[fb + p] : 0.0;
+    };
+    load_arcs(k0);
+    load_masks(k0);
+    for (int k = k0; k < k1; ++k) {
+        const size_t fb = ((size_t)l * kall + k) * gall;
+        // phase 1 of the level below, the last reader of s_q and s_g, lies before the last barrier
 #pragma unroll
-            for (int d = 0; d < 3; ++d) s_g[d * n_in + s] = ok ? A.grad[d * plane + fb + p] : 0.0;
+        for (int u = 0; u < NSTG; ++u) {
+            const int s = tid + u * RCH;
+            if (s < n_in) {
+                s_q[s] = stg[u][0];
+#pragma unroll
+                for (int d = 0; d < 3; ++d) s_g[d * n_in + s] = stg[u][1 + d];
+            }
         }
         __syncthreads();
         // phase 1: the two reconstructions of each arc (GRD_xc(g,k,l,a,d) at (d*3+a)*plane)
@@ -245,6 +268,7 @@ __global__ void __launch_bounds__(RCH) remap_kernel(RemapArgs A)
                 s_a[(3 + a) * n_o + s] = qn;
             }
         }
+        if (k + 1 < k1) load_arcs(k + 1);
         __syncthreads();
         // phase 2: my faces, each by its own mask
         if (active) {
@@ -262,7 +286,8 @@ __global__ void __launch_bounds__(RCH) remap_kernel(RemapArgs A)
             if (f5) stream_store(&A.q_a[4 * plane + fb + g], cm[4] * s_a[1 * n_o + o5] + (1.0 - cm[4]) * s_a[4 * n_o + o5]);
             if (f6) stream_store(&A.q_a[5 * plane + fb + g], cm[5] * s_a[2 * n_o + o6] + (1.0 - cm[5]) * s_a[5 * n_o + o6]);
         }
-        __syncthreads();  // the tiles are restaged for the next level
+        if (k + 1 < k1) load_masks(k + 1);
+        // phase 1 of the next level writes s_a behind that level's first barrier
     }
 }
 
@@ -382,9 +407,10 @@ int launch_remap(nicam_ctx c, double *q_a, double *q_a_pl, const double *q, cons
     A.have_pl = D.have_pl && q_a_pl;
     A.nchunk = (D.gall + RCH - 1) / RCH;
     const long base = (long)A.nchunk * D.lall;
-    int nkr = (int)((4096 + base - 1) / base);  // enough work-groups to fill the chip
-    nkr = std::max(1, std::min(nkr, D.kall));
-    A.kper = (D.kall + nkr - 1) / nkr;
+    // two work-groups per CU (registers).  us at kper: 18x18x42x40 38 at 1, 31 at 4, 26.4 at 7 (one round), 41 at 14;
+    // 34x34x42x10 26 at 1, 21 at 5 (one round), 27 at 8; 34x34x78x40 203 at 1, 181 at 8, 199 at 14; 66x66x98x40 911 at
+    // 1, 798 at 10, 829 at 26 (with many rounds the short marches stay ahead, hence the cap)
+    A.kper = level_split(base, D.kall, 512, 10);
     A.nkr = (D.kall + A.kper - 1) / A.kper;
     const long nmain = base * A.nkr;
     const long npole = A.have_pl ? ((long)D.kall * kLallPl + RCH - 1) / RCH : 0;
@@ -392,7 +418,8 @@ int launch_remap(nicam_ctx c, double *q_a, double *q_a_pl, const double *q, cons
     A.nmain = (int)nmain;
     const int n_in = RCH + 2 * D.gall_1d + 2, n_o = RCH + D.gall_1d + 1;
     const size_t lds = sizeof(double) * (7 * (size_t)n_in + 6 * (size_t)n_o);
-    hipLaunchKernelGGL(remap_kernel, dim3((unsigned)(nmain + npole)), dim3(RCH), lds, c->stream, A);
+    hipLaunchKernelGGL(n_in <= 2 * RCH ? remap_kernel<2> : remap_kernel<3>, dim3((unsigned)(nmain + npole)), dim3(RCH),
+                       lds, c->stream, A);
     NICAM_HIP(hipGetLastError());
     return NICAM_OK;
 }

@@ -377,19 +377,7 @@ int hflux_launch(void (*const k[4])(Arg), int v, long nblk, size_t lds, hipStrea
 template <class T>
 int hflux_kper(long base, int kall)
 {
-    const long slots = sizeof(T) == 8 ? 512 : 1024;
-    const int cap = sizeof(T) == 8 ? kall : std::min(kall, 14);
-    int best = 1;
-    double cost = 0.0;
-    for (int kper = 1; kper <= cap; ++kper) {
-        const long n = base * ((kall + kper - 1) / kper);
-        const double t = (double)((n + slots - 1) / slots) * (kper + 1.5);
-        if (kper == 1 || t <= cost) {
-            cost = t;
-            best = kper;
-        }
-    }
-    return best;
+    return sizeof(T) == 8 ? level_split(base, kall, 512, kall) : level_split(base, kall, 1024, 14);
 }
 
 // The launch arguments of one grid: nblk work-groups, lds bytes, nst the

@@ -181,6 +181,26 @@ int hip_fail(hipError_t e, const char *what);
         if (e_ != hipSuccess) return ::nicam::hip_fail(e_, #call); \
     } while (0)
 
+// Levels per work-group, at most cap, of a kernel whose work-groups march up a
+// range of levels: base columns of work-groups over kall levels, slots of them
+// on the chip at a time, each paying about one and a half levels to start.  The
+// launch costs rounds * (levels + 1.5); the least of that, the longer march on
+// a tie.
+inline int level_split(long base, int kall, long slots, int cap)
+{
+    int best = 1;
+    double cost = 0.0;
+    for (int kper = 1; kper <= std::min(cap, kall); ++kper) {
+        const long n = base * ((kall + kper - 1) / kper);
+        const double t = (double)((n + slots - 1) / slots) * (kper + 1.5);
+        if (kper == 1 || t <= cost) {
+            cost = t;
+            best = kper;
+        }
+    }
+    return best;
+}
+
 // Hardware dispatch sends work-group b to XCD b % 8, and each XCD has its own
 // L2.  For a launch of n work-groups whose neighbours in logical order share
 // data (halo rows, the level above and below), this maps the hardware index
