@@ -589,12 +589,10 @@ int launch_diffusion(nicam_ctx c, double *dscl, double *dscl_pl, const double *s
     A.have_pl = D.have_pl;
     A.nchunk = (D.gall + CHUNK - 1) / CHUNK;
     const long base = (long)A.nchunk * D.lall;
-    // about 1024 work-groups: longer level marches read the coefficients fewer times (gl7: two ranges
-    // of 49 levels 290 us, three of 33 298 us, six of 17 337 us)
-    int nkr = (int)((1024 + base - 1) / base);
-    nkr = std::max(1, std::min(nkr, D.kall));
-    if (c->tune.diff_kper > 0) nkr = (D.kall + c->tune.diff_kper - 1) / c->tune.diff_kper;
-    A.kper = (D.kall + nkr - 1) / nkr;
+    // two work-groups per CU (registers).  us at levels per work-group: 18x18x42x40 21.8 at 3, 16.3 at 7 (one round),
+    // 24.7 at 14; 34x34x78x40 81 at 13, 75 at 8; 66x66x98x40 289 at 49 (three rounds), 291 at 33, 318 at 10, 352 at 98;
+    // 130x130x40x10 143 at 20, 132 at 14
+    A.kper = c->tune.diff_kper > 0 ? std::min(c->tune.diff_kper, D.kall) : level_split(base, D.kall, 512, D.kall);
     A.nkr = (D.kall + A.kper - 1) / A.kper;
     const long nmain = base * A.nkr;
     const long npole = dscl_pl ? (D.kall * kLallPl + CHUNK - 1) / CHUNK : 0;
@@ -658,19 +656,18 @@ int launch_divdamp(nicam_ctx c, double *const out[3], double *const out_pl[3], c
     A.nchunk = (D.gall + CHUNK - 1) / CHUNK;
     const int nlev = D.kall - 2;  // kmin..kmax
     const long base = (long)A.nchunk * D.lall;
-    // about 1024 work-groups (gl7: two ranges of 48 levels 566 us, three of 32 603 us)
-    int nkr = (int)((1024 + base - 1) / base);
-    nkr = std::max(1, std::min(nkr, nlev));
-    if (c->tune.ddmp_kper > 0) nkr = (nlev + c->tune.ddmp_kper - 1) / c->tune.ddmp_kper;
-    A.kper = (nlev + nkr - 1) / nkr;
+    const int n_x = D.gall_1d + 1;
+    const bool small = 2 * n_x <= CHUNK;  // the cells below and above the chunk fit one extra slot
+    // two work-groups per CU, one where the third slot's registers leave room for no more.  us at levels per
+    // work-group: 18x18x42x40 32.8 at 3, 24.4 at 7 (one round), 33 at 14; 51x51x61x7 46.5 at 5, 36.5 at 10 (one round),
+    // 51 at 20; 66x66x98x40 566 at 48 (three rounds), 600 at 32, 617 at 10, 687 at 96; 130x130x40x10 457 at 19, 430 at 13
+    A.kper = c->tune.ddmp_kper > 0 ? std::min(c->tune.ddmp_kper, nlev) : level_split(base, nlev, small ? 512 : 256, nlev);
     A.nkr = (nlev + A.kper - 1) / A.kper;
     const long nmain = base * A.nkr;
     const long npole = out_pl[0] ? (D.kall * kLallPl + CHUNK - 1) / CHUNK : 0;
     if (nmain + npole > 0x7fffffffL) return fail(NICAM_ERR_ARG, "grid too large for one launch");
     A.nmain = (int)nmain;
-    const int n_x = D.gall_1d + 1;
     const size_t lds = sizeof(double) * (5 * (CHUNK + 2 * n_x) + 2 * (CHUNK + n_x) + 18 * n_x);
-    const bool small = 2 * n_x <= CHUNK;  // the cells below and above the chunk fit one extra slot
     const void *fn = small ? (const void *)ddmp_kernel<2> : (const void *)ddmp_kernel<3>;
     if (lds > 64 * 1024) NICAM_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     if (small)

@@ -236,6 +236,14 @@ def test_gpu_glue_kernels_match_oracle(gpu, oracle, gl, rl, kall):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("gl,rl,kall", [(7, 0, 11), (5, 1, 23), (3, 0, 4)])
+def test_gpu_glue_kernels_match_oracle_over_level_ranges(gpu, oracle, gl, rl, kall):
+    """Regions wide enough for a third staged cell per work-item, several level
+    ranges with a shorter last one, the fewest levels."""
+    test_gpu_glue_kernels_match_oracle(gpu, oracle, gl, rl, kall)
+
+
+@pytest.mark.gpu
 def test_gpu_chained_step_matches_oracle(gpu, oracle):
     """flux -> courant -> gradient -> halo fill of the gradient -> remap ->
     limiter with its own Qout exchange -> update, all on the device through
