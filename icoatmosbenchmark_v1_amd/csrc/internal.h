@@ -188,12 +188,13 @@ int hip_fail(hipError_t e, const char *what);
 // a tie.
 inline int level_split(long base, int kall, long slots, int cap)
 {
-    int best = 1;
+    int best = 0;
     double cost = 0.0;
-    for (int kper = 1; kper <= std::min(cap, kall); ++kper) {
-        const long n = base * ((kall + kper - 1) / kper);
-        const double t = (double)((n + slots - 1) / slots) * (kper + 1.5);
-        if (kper == 1 || t <= cost) {
+    for (int kper = std::min(cap, kall); kper >= 1; --kper) {
+        const int nkr = (kall + kper - 1) / kper;
+        kper = (kall + nkr - 1) / nkr;  // the shortest march of as many ranges
+        const double t = (double)((base * nkr + slots - 1) / slots) * (kper + 1.5);
+        if (best == 0 || t < cost) {
             cost = t;
             best = kper;
         }
