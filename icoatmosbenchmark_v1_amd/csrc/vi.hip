@@ -277,6 +277,10 @@ __global__ void __launch_bounds__(BLOCK_REG) vi_kernel_reg(ViArgsT<Src> A)
 constexpr int NW = 4, BLOCK_CO = 64 * NW;
 constexpr int CB = 4;   // levels of source loads in flight per wave
 constexpr int CD = 16;  // levels of factors in flight in the recurrences
+// 64 columns of a level row end inside cache lines that the next 64 share: COWIN
+// consecutive work-groups run on one XCD (gl7 step 1802 -> 1745 us; 4: 1787, an
+// eighth of the launch to each XCD: 1816)
+constexpr int COWIN = 16;
 constexpr int CG = 16;  // levels of the final scaling in flight per wave
 
 template <class Src>
@@ -414,7 +418,7 @@ template <class Src>
 __global__ void __launch_bounds__(BLOCK_CO) vi_kernel_coop(ViArgsT<Src> A)
 {
     extern __shared__ double s_w[];
-    vi_coop_block<Src>(A, blockIdx.x, s_w);
+    vi_coop_block<Src>(A, xcd_windowed(blockIdx.x, gridDim.x, COWIN), s_w);
 }
 
 static_assert(BLOCK_CO == 256 && BLOCK_FAC == 256, "vi_group_kernel serves both");
@@ -437,7 +441,7 @@ __global__ void __launch_bounds__(256) vi_group_kernel(ViGroup<Src> G)
     const ViArgsT<Src> &A = G.a[n];
     if constexpr (COOP) {
         extern __shared__ double s_w[];
-        vi_coop_block<Src>(A, b - G.off[n], s_w);
+        vi_coop_block<Src>(A, xcd_windowed(b - G.off[n], G.off[n + 1] - G.off[n], COWIN), s_w);
     } else {
         column_run<BLOCK_FAC>(A, b - G.off[n], [&](const ViFieldT<Src> &F, size_t base, size_t s) {
             NoGamma gam;
