@@ -544,8 +544,8 @@ int launch_vi_t(nicam_ctx c, double *w, double *w_pl, const Src *w0, const Src *
     int variant = c->tune.vi_variant;
     const bool reg_ok = (D.kall == 42 || D.kall == 98);
     if (((variant == 3 || variant == 4) && !reg_ok) || (variant == 5 && D.kall > kMaxCoop)) variant = 0;
-    // measured with the v-limiter (us; 5 against the best other): 40 x 66x66 x 98 FP64 518 against 533 (4), FP32
-    // inputs 346 against 400 (4); x 97 FP64 512 against 640 (2); 40 x 34x34 x 58 93 against 123 (2); 7 x 51x51 x 61
+    // measured with the v-limiter (us; 5 against the best other): 40 x 66x66 x 98 FP64 506 against 533 (4), FP32
+    // inputs 332 against 400 (4); x 97 FP64 512 against 640 (2); 40 x 34x34 x 58 93 against 123 (2); 7 x 51x51 x 61
     // 57.6 against 98.7 (2); 12x12 x 98 31.3 against 32.6 (4).  At 42 levels the registers hold the column at two
     // waves per SIMD and 4 is as fast or faster (130x130 37.3 against 38.7, 10 x 66x66 68.1 against 71.9).
     if (variant == 0) variant = D.kall == 42 ? 4 : (D.kall <= kMaxCoop ? 5 : 2);
