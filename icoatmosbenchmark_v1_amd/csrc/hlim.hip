@@ -55,6 +55,21 @@ __device__ __forceinline__ float sign_half(float x) { return copysignf(0.5f, x);
 __device__ __forceinline__ double tabs(double x) { return fabs(x); }
 __device__ __forceinline__ float tabs(float x) { return fabsf(x); }
 
+// A face value clamped into the inflow bounds of its two sides (side 1 where
+// c = 1, side 2 where c = 0), then into the allowable range of the cell it
+// flows out to (HLIM:377-410).  The reference's compare-and-select form hands a
+// NaN first operand on, an instruction takes the bound instead: NaN is
+// therefore restored where the face is NaN, and where the first line makes one
+// (0 * inf, from infinite faces, tracers or masks) that the second would clamp.
+template <class T>
+__device__ __forceinline__ T clamp_face(T qa, T c, T in_mn1, T in_mx1, T in_mn2, T in_mx2, T out_mn1, T out_mx1,
+                                        T out_mn2, T out_mx2)
+{
+    const T in = (c)*hw_min(hw_max(qa, in_mn1), in_mx1) + (T(1) - c) * hw_min(hw_max(qa, in_mn2), in_mx2);
+    const T out = (c)*hw_max(hw_min(in, out_mx1), out_mn1) + (T(1) - c) * hw_max(hw_min(in, out_mx2), out_mn2);
+    return __builtin_isunordered(qa, in) ? T(__builtin_nan("")) : out;
+}
+
 template <class T>
 struct HlimArgs {
     T *q_a;          // (gall,kall,lall,6) inout
@@ -317,9 +332,7 @@ __device__ __forceinline__ void hlim_block(const HlimArgs<T> &A, int b)
                 const T qo_max_n = PF ? pre_qpn[m][1] : Qpost[plane + fb + nb[m]];
                 T qa = PF ? pre_qa[m] : ld_once(&q_a[(size_t)m * plane + fb + g]);
                 const T qa_in = qa;
-                qa = (c)*hw_min(hw_max(qa, in_mn_s[m]), in_mx_s[m]) + (T(1) - c) * hw_min(hw_max(qa, in_mn_n), in_mx_n);
-                qa = (c)*hw_max(hw_min(qa, qo_max_n), qo_min_n) + (T(1) - c) * hw_max(hw_min(qa, qo_max_c), qo_min_c);
-                qa = keep_nan(qa_in, qa);
+                qa = clamp_face(qa_in, c, in_mn_s[m], in_mx_s[m], in_mn_n, in_mx_n, qo_min_n, qo_max_n, qo_min_c, qo_max_c);
                 bits |= (qa != qa_in ? 1u : 0u) << m;
 #if NICAM_HLIM_STORE == 2
                 q_a[(size_t)m * plane + fb + g] = qa;
@@ -439,9 +452,7 @@ __device__ void hlim_pole(const HlimArgs<T> &A0, int t, int tr)
         const T c = A.cmask_pl[fb + v];
         T qa = A.q_a_pl[fb + v];
         const T qa_in = qa;
-        qa = (c)*hw_min(hw_max(qa, mn1), mx1) + (T(1) - c) * hw_min(hw_max(qa, mn2), mx2);
-        qa = (c)*hw_max(hw_min(qa, A.Qpost_pl[plane + fb + v]), A.Qpost_pl[fb + v]) + (T(1) - c) * hw_max(hw_min(qa, pn_max), pn_min);
-        qa = keep_nan(qa_in, qa);
+        qa = clamp_face(qa_in, c, mn1, mx1, mn2, mx2, A.Qpost_pl[fb + v], A.Qpost_pl[plane + fb + v], pn_min, pn_max);
         A.q_a_pl[fb + v] = qa;
         if (A.mask_pl) A.mask_pl[fb + v] = (qa != qa_in) ? 1 : 0;
     }

@@ -231,8 +231,9 @@ __device__ __forceinline__ long xcd_windowed(long b, long n, long unit)
 // selects: a third of the kernel's vector instructions (1011 -> 798 in FP64;
 // gl7 649 -> 635 us, in exchange mode at gl6 160 -> 156 us).  The two differ
 // only where a is NaN (the select keeps it, the instruction returns b) and in
-// which of two zeros of opposite sign is returned; keep_nan restores the first
-// where it reaches a result.
+// which of two zeros of opposite sign is returned.  The limiter restores NaN
+// where the select form would have handed it on: at an arc's first value
+// (keep_nan) and in its clamp (clamp_face, which tells what can make one there).
 // (Written as instructions: the compiler's fmin first quiets every operand that
 // comes from memory, one more instruction each.)
 #define NICAM_HW_MINMAX(name, T, op)                                \
