@@ -353,6 +353,7 @@ __device__ __forceinline__ void hlim_block(const HlimArgs<T> &A, int b)
 template <class T, bool MULTI, bool PRE = false, int TW = MAXI_TILE>
 __global__ void __launch_bounds__(CHUNK) hlim_kernel(HlimArgs<T> A)
 {
+    minmax_skip_any_nan();
     hlim_block<T, MULTI, PRE, TW>(A, blockIdx.x);
 }
 
@@ -367,6 +368,7 @@ struct HlimGroup {
 template <class T>
 __global__ void __launch_bounds__(CHUNK) hlim_group_kernel(HlimGroup<T> G)
 {
+    minmax_skip_any_nan();
     const int b = blockIdx.x;
     int n = 0;
     while (n + 1 < G.n && b >= G.off[n + 1]) ++n;

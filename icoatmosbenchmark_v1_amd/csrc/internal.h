@@ -263,6 +263,17 @@ NICAM_HW_MINMAX(hw_max, float, "v_max_f32")
 NICAM_HW_MINMAX3(hw_min3, hw_min, "v_min3_f32")
 NICAM_HW_MINMAX3(hw_max3, hw_max, "v_max3_f32")
 #undef NICAM_HW_MINMAX3
+// The select form skips a NaN second operand, signalling or quiet.  With the
+// wave's MODE.IEEE bit set, as kernels start, v_min and v_max return NaN for a
+// signalling one (an array filled with it to catch unset cells, say); with the
+// bit clear they skip it too.  Nothing else here depends on the bit: it only
+// decides whether signalling NaNs are quieted.  Called first in a kernel that
+// uses the functions above.
+__device__ __forceinline__ void minmax_skip_any_nan()
+{
+    constexpr int kMode = 1, kIeeeBit = 9;
+    __builtin_amdgcn_s_setreg(kMode | kIeeeBit << 6, 0);  // hwreg(MODE, 9, 1) = 0
+}
 // r, or a where a is NaN
 template <class T>
 __device__ __forceinline__ T keep_nan(T a, T r) { return a == a ? r : a; }

@@ -222,22 +222,28 @@ def test_hlim_keeps_nan_and_infinity_where_the_reference_form_does(gpu, oracle, 
         np.testing.assert_array_equal(got[k], want[k], err_msg=k)
 
 
-NONFINITE = {"inf": (np.inf, -np.inf), "nan": (np.nan, np.inf, -np.inf)}
+NONFINITE = {"inf": (np.inf, -np.inf), "nan": (np.nan, np.inf, -np.inf), "snan": ("signalling", np.inf, -np.inf)}
 
 
 def _plant(a, idx, v):
-    a.reshape(-1)[idx] = v
+    """a.flat[idx] = v; a signalling NaN by its bits, which a float would not keep."""
+    if v == "signalling":
+        u, bits = (np.uint64, 0x7FF0000000000001) if a.dtype == np.float64 else (np.uint32, 0x7F800001)
+        a.reshape(-1).view(u)[idx] = bits
+    else:
+        a.reshape(-1)[idx] = v
 
 
+@pytest.mark.filterwarnings("ignore:invalid value encountered in cast")  # a signalling NaN widened for the oracle
 @pytest.mark.parametrize("values", sorted(NONFINITE))
 @pytest.mark.parametrize("mode", ["post", "exchange", "batch"])
 @pytest.mark.parametrize("dtype", [np.float64, np.float32], ids=["f64", "f32"])
 def test_hlim_nonfinite_tracers_and_faces_together(gpu, oracle, dtype, mode, values):
     """A blown-up field: tracers and face values around the same arcs not
     finite at once.  Between the clamp's two lines 0 * inf makes a NaN out of
-    inputs none of which is one, and the compare-and-select form keeps it.
-    Qout_post finite, the library's own exchange of Qout_prev, and two tracers
-    at once.
+    inputs none of which is one, and the compare-and-select form keeps it;
+    a min or max takes a signalling NaN as it takes a quiet one.  Qout_post
+    finite, the library's own exchange of Qout_prev, and two tracers at once.
     In FP32 the oracle computes in FP64 on the rounded inputs: with Qout_post
     given, a face is one of the inputs and equal; ranges and exchanged faces
     are NaN at the same places."""
