@@ -493,9 +493,22 @@ class TracerStep:
     # -- the step ----------------------------------------------------------------
     def face_values(self, q, q_pl, xc, xc_pl, cm, cm_pl, ch, ch_pl):
         """One tracer's limited face values: gradient, exchange, remap, the
-        limiter's allowable range, its exchange, the clamp."""
-        return FaceValues.apply(self.ctx, self.cg, self.cg_pl, self.X, self.X_pl, self.d, self.d_pl, cm, cm_pl, q, q_pl,
-                                xc, xc_pl, ch, ch_pl)
+        limiter's allowable range, its exchange, the clamp.  One node, unless
+        gradient, halo or remap has been replaced (in a subclass, on the
+        instance or on the class): then the stages one by one."""
+        if self._own_stages():
+            return FaceValues.apply(self.ctx, self.cg, self.cg_pl, self.X, self.X_pl, self.d, self.d_pl, cm, cm_pl, q,
+                                    q_pl, xc, xc_pl, ch, ch_pl)
+        grad, grad_pl = self.gradient(q, q_pl)
+        grad, grad_pl = self.halo(grad, grad_pl)
+        q_a, q_a_pl = self.remap(q, q_pl, grad, grad_pl, cm, cm_pl, xc, xc_pl)
+        return HorizontalLimiter.apply(self.ctx, q_a.contiguous(), q_a_pl.contiguous(), q.contiguous(), q_pl.contiguous(),
+                                       self.d, self.d_pl, ch, ch_pl, cm, cm_pl)
+
+    def _own_stages(self) -> bool:
+        own = lambda m, f: getattr(m, "__func__", None) is f and m.__self__ is self  # noqa: E731
+        return (own(self.gradient, _GRADIENT) and own(self.remap, _REMAP) and type(self.halo) is HaloExchange
+                and HaloExchange.__call__ is _EXCHANGE and self.halo.nctx is self.ctx)
 
     def __call__(self, q, q_pl, rhog, rhog_pl, recompute_tracers: bool = False):
         """One step.  recompute_tracers: each tracer's face values are
@@ -536,3 +549,7 @@ class TracerStep:
         """1/2 sum of q^2 over the inner cells, the pole centres and kmin..kmax."""
         w = self.inner.to(q.dtype) * self.kin
         return 0.5 * ((q * q) * w).sum() + 0.5 * ((q_pl[..., 0] * q_pl[..., 0]) * self.kin[:, 0]).sum()
+
+
+# the stages FaceValues stands for
+_GRADIENT, _REMAP, _EXCHANGE = TracerStep.gradient, TracerStep.remap, HaloExchange.__call__
