@@ -48,6 +48,8 @@ struct VlimArgs {
     T eps, big;
     int ntr;          // tracers
     long ts, tps;     // tracer strides of the regular and pole fields
+    unsigned ncol;    // columns, the poles' last
+    unsigned unit, win, wfull;  // work-groups of a column block, of a window of 8 * WIN blocks, of all whole windows
     uint32_t *mask, *mask_pl;  // clip bits (masked variant only; kc = 8)
 };
 
@@ -180,35 +182,34 @@ __device__ __forceinline__ uint32_t vlim_run_kc(T *__restrict__ q_h, const T *__
 // tracer.  The tracers and runs of one column block are consecutive
 // work-groups on one XCD: the tracers read the same ck and d, and each run
 // also reads the two levels below it, which the run below has just brought
-// into that XCD's L2.  Each XCD takes WIN column blocks at a time, next to the
-// other XCDs' (xcd_windowed): 154 us at gl7 FP64 against 163 us with an eighth
-// of the launch to each XCD; eight FP32 tracers on four grids 1.15 ms against
-// 1.25 ms with four tracers per work-item and their levels loaded one at a
-// time.  KC > 0: runs of KC levels known at compile time
-// (vlim_run_kc); 0: of A.kc levels (vlim_run).
+// into that XCD's L2.  (Eight FP32 tracers on four grids 1.15 ms, against 1.25
+// ms with four tracers per work-item and their levels loaded one at a time.)
+// KC > 0: runs of KC levels known at compile time (vlim_run_kc); 0: of A.kc
+// levels (vlim_run).
 // MASK: with runs of eight faces, a byte of the 32-face mask words each (face
 // p is bit p % 32 of word p / 32); the last run clears its word's other bytes.
 // (18x18x42x40, where runs of a whole word leave 102 work-groups: 58 -> 12 us.)
 template <class T, int KC, bool MASK = false>
-__device__ __forceinline__ void vlim_block(const VlimArgs<T> &A, long blk)
+__device__ __forceinline__ void vlim_block(const VlimArgs<T> &A, unsigned blk)
 {
-    const long ncol_reg = (long)A.gall * A.lall;
-    const long ncol = ncol_reg + (A.have_pl ? (long)A.gall_pl * kLallPl : 0);
-    const long ncb = (ncol + BLOCK - 1) / BLOCK;  // column blocks
-    const int unit = A.nrun * A.ntr;
-    const long L = xcd_windowed(blk, ncb * unit, WIN * unit);
-    const long cb = L / unit;
-    const int ru = (int)(L - cb * unit), run = ru / A.ntr, tr = ru - run * A.ntr;
-    const long col = cb * BLOCK + threadIdx.x;
-    if (col >= ncol) return;
+    // every argument at once: behind the branches below they would come one batch after the other
+    asm volatile("" ::"s"(A.q_h), "s"(A.q), "s"(A.d), "s"(A.ck), "s"(A.gall), "s"(A.kall), "s"(A.lall), "s"(A.ncol),
+                 "s"(A.unit), "s"(A.win), "s"(A.wfull), "s"(A.ntr), "s"(A.ts), "s"(A.eps), "s"(A.big));
+    const unsigned ncol_reg = (unsigned)A.gall * A.lall;
+    const unsigned w = blk / A.win, r = blk - w * A.win;
+    const unsigned L = blk < A.wfull ? w * A.win + (r & 7) * (A.win >> 3) + (r >> 3) : blk;
+    const unsigned cb = L / A.unit, ru = L - cb * A.unit;
+    const int run = A.ntr == 1 ? ru : ru / A.ntr, tr = ru - run * A.ntr;
+    const unsigned col = cb * BLOCK + threadIdx.x;
+    if (col >= A.ncol) return;
     const int kmin = 1, kmax = A.kall - 2;  // 0-based
     const int kc = KC > 0 ? KC : A.kc;
     const int kb = kmin + 1 + run * kc;
     const int ke = min(kmax + 1, kb + kc);
     if (kb >= ke) return;
-    auto go = [&](auto pole, T *q_h, const T *q, const T *d, const T *ck, long t, int gall, int lall, uint32_t *mask) {
+    auto go = [&](auto pole, T *q_h, const T *q, const T *d, const T *ck, unsigned t, int gall, int lall, uint32_t *mask) {
         constexpr bool POLE = decltype(pole)::value;
-        const int g = (int)(t % gall), l = (int)(t / gall);
+        const unsigned l = t / gall, g = t - l * gall;
         const size_t base = (size_t)l * A.kall * gall + g;
         const size_t ck2 = (size_t)gall * A.kall * lall;
         if constexpr (KC > 0) {
@@ -297,8 +298,20 @@ int vlim_make_args(nicam_ctx c, VlimArgs<T> &A, long &nblk, T *q_h, T *q_h_pl, c
     A.kc = kc;
     A.nrun = (nlev + kc - 1) / kc;
     const long ncol = (long)D.gall * D.lall + (D.have_pl ? (long)D.gall_pl * kLallPl : 0);
-    nblk = (ncol + BLOCK - 1) / BLOCK * A.nrun * ntr;
-    if (nblk > 0x7fffffffL) return fail(NICAM_ERR_ARG, "grid too large for one launch");
+    const long ncb = (ncol + BLOCK - 1) / BLOCK, unit = (long)A.nrun * ntr;  // column blocks, work-groups of each
+    nblk = ncb * unit;
+    // 2^32 columns of four levels are more than the device's memory
+    if (nblk > 0x7fffffffL || ncol > 0xffffffffL) return fail(NICAM_ERR_ARG, "grid too large for one launch");
+    A.ncol = (unsigned)ncol;
+    A.unit = (unsigned)unit;
+    // Fields beyond the Infinity Cache (256 MB; q, q_h and its result per tracer, ck's two planes and d): each XCD takes
+    // WIN column blocks at a time, next to the other XCDs' (gl7 FP64 154 us against 163 with an eighth of the launch to
+    // each XCD, FP32 67 against 71; 130x130x42x40 250 against 270).  In the cache: an eighth of the launch
+    // (90x90x97x3 20.2 us against 22.0 in windows, FP32 12.9 against 13.4; 66x66x42x40 FP32 27.7 and 28.7).
+    const bool large = sizeof(T) * (3.0 * ntr + 3.0) * ncol * D.kall > 256e6;
+    const long win = large ? 8 * WIN * unit : nblk / 8 * 8, nwin = win > 0 ? nblk / win : 0;
+    A.win = nwin > 0 ? (unsigned)win : 8;
+    A.wfull = (unsigned)(nwin * win);
     return NICAM_OK;
 }
 

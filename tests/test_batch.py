@@ -101,8 +101,8 @@ def test_gpu_batched_limiters_equal_single_tracer_calls(gpu, single, grid):
 @pytest.mark.gpu
 @pytest.mark.parametrize("ntr,kall,kc", [(3, 10, 0), (1, 11, 0), (2, 9, 3), (3, 4, 0)])
 def test_gpu_batched_vertical_limiter_maps_every_work_group(gpu, oracle, ntr, kall, kc):
-    """Enough column blocks (182 with the poles) for several full windows of
-    the XCD mapping and a remainder, every tracer against the oracle."""
+    """A launch of several hundred work-groups, not a multiple of the eight
+    XCDs, every tracer against the oracle."""
     import torch
 
     spec = synth.GridSpec(34, kall, 40, have_pl=True, seed=66)
@@ -120,6 +120,40 @@ def test_gpu_batched_vertical_limiter_maps_every_work_group(gpu, oracle, ntr, ka
         want = oracle.vertical_limiter_thuburn(spec, vs[t])
         for k in ("q_h", "q_h_pl"):
             assert np.array_equal(st[k][t].cpu().numpy(), want[k]), (t, k)
+    ctx.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("single,ntr", [(False, 4), (True, 8)], ids=["f64", "f32"])
+def test_gpu_batched_vertical_limiter_beyond_the_cache(gpu, oracle, single, ntr):
+    """Fields larger than the Infinity Cache: the XCDs take windows of column
+    blocks (793 blocks and the poles: 24 windows and a remainder); every tracer
+    as in a call of its own, whose launch is the other mapping, the first
+    against the oracle."""
+    import torch
+
+    spec = synth.GridSpec(130, 12, 12, have_pl=True, seed=67)
+    case = synth.make_case(spec, have_sgp=[1] + [0] * 11)
+    ctx = drivers.setup_context(spec, case["geo"])
+    dt, sfx = (torch.float32, "_f32") if single else (torch.float64, "")
+    v = {k: torch.from_numpy(np.ascontiguousarray(x)).to(gpu, dt) for k, x in case["vlim"].items()}
+    q = torch.stack([torch.roll(v["q"], 5 * t, -1) for t in range(ntr)]).contiguous()
+    q_h = torch.stack([torch.roll(v["q_h"], 3 * t, -1) for t in range(ntr)]).contiguous()
+    q_pl, q_h_pl = (v[k].expand((ntr,) + spec.shape_pl).contiguous() for k in ("q_pl", "q_h_pl"))
+    assert q.element_size() * (3 * ntr + 3) * q[0].numel() > 256e6
+    fixed = [v[k] for k in ("d", "d_pl", "ck", "ck_pl")]
+    want = []
+    for t in range(ntr):
+        a, a_pl = q_h[t].clone(), q_h_pl[t].clone()
+        getattr(ctx, "vertical_limiter_thuburn" + sfx)(a, a_pl, q[t], q_pl[t], *fixed)
+        want.append((a, a_pl))
+    getattr(ctx, "vertical_limiter_thuburn_batch" + sfx)(ntr, q_h, q_h_pl, q, q_pl, *fixed)
+    for t in range(ntr):
+        assert torch.equal(q_h[t], want[t][0]) and torch.equal(q_h_pl[t], want[t][1]), t
+    if not single:
+        ref = oracle.vertical_limiter_thuburn(spec, case["vlim"])
+        for k, x in (("q_h", q_h), ("q_h_pl", q_h_pl)):
+            assert np.array_equal(x[0].cpu().numpy(), ref[k]), k
     ctx.close()
 
 
