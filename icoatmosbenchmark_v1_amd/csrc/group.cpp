@@ -283,7 +283,8 @@ int nicam_group_autotune(nicam_group g, int ntr, const nicam_tracer_step_f32 *gr
     for (size_t i = 0; i < g->ctxs.size(); ++i) {
         const nicam_ctx c = g->ctxs[i];
         const nicam_tracer_step_f32 &p = grids[i];
-        const std::string key = "nicam_tt-tune v1 " + tune_key(c, ntr) + " ";
+        // the version counts the kernels' generations: what was best for another one's is timed again
+        const std::string key = "nicam_tt-tune v2 " + tune_key(c, ntr) + " ";
         bool found = false;
         for (const std::string &ln : cache) {
             int kper = 0, kch = 0;

@@ -221,6 +221,29 @@ def _assert_equal_outputs(S, want):
 
 
 @pytest.mark.gpu
+def test_gpu_autotune_times_again_what_another_generation_of_kernels_chose(gpu, tmp_path):
+    """A cache line of the first version of the kernels is left in the file
+    and not applied; the line timed now is the one read back."""
+    from icoatmosbenchmark_v1_amd.group import Group, batched_state
+
+    spec, case = _grid(GRIDS[0])
+    ctx = drivers.setup_context(spec, case["geo"], case["vi"])
+    grp = Group([ctx])
+    states = [batched_state(spec, case, 2, device=gpu)]
+    cache = tmp_path / "tune.txt"
+    assert grp.autotune(2, states, 360.0, 60.0, str(cache)) > 0
+    line = cache.read_text()
+    old = line.replace(" v2 ", " v1 ")
+    assert old != line
+    cache.write_text(old)
+    assert grp.autotune(2, states, 360.0, 60.0, str(cache)) > 0
+    assert cache.read_text().splitlines()[0] == old.strip() and cache.read_text().count("\n") == 2
+    assert grp.autotune(2, states, 360.0, 60.0, str(cache)) == 0
+    grp.close()
+    ctx.close()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("kcs", [(2, 0, 0), (8, 4, 5), (16, 2, 8), (3, 3, 1000)])
 def test_gpu_group_step_with_tuned_runs_of_the_vertical_limiter(gpu, kcs):
     """Grids of one launch with different run lengths, as an autotuner or its
