@@ -408,7 +408,7 @@ int hflux_make_args(nicam_ctx c, HfluxArgs<T> &A, long &nblk, size_t &lds, int &
     A.eps = eps;
     A.nchunk = (D.gall + CHUNK - 1) / CHUNK;
     const long base = (long)A.nchunk * D.lall;
-    A.kper = c->tune.hflux_kper > 0 ? std::min(c->tune.hflux_kper, D.kall) : hflux_kper<T>(base, D.kall);
+    A.kper = c->tune.hflux_kper > 0 ? even_split(D.kall, c->tune.hflux_kper) : hflux_kper<T>(base, D.kall);
     A.nkr = (D.kall + A.kper - 1) / A.kper;
     const long nmain = base * A.nkr;
     const long npole = D.have_pl ? (D.kall * kLallPl + CHUNK - 1) / CHUNK : 0;

@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "nicam_tt.h"
+#include "split.h"
 
 namespace nicam {
 
@@ -180,27 +181,6 @@ int hip_fail(hipError_t e, const char *what);
         hipError_t e_ = (call);                                  \
         if (e_ != hipSuccess) return ::nicam::hip_fail(e_, #call); \
     } while (0)
-
-// Levels per work-group, at most cap, of a kernel whose work-groups march up a
-// range of levels: base columns of work-groups over kall levels, slots of them
-// on the chip at a time, each paying about one and a half levels to start.  The
-// launch costs rounds * (levels + 1.5); the least of that, the longer march on
-// a tie.
-inline int level_split(long base, int kall, long slots, int cap)
-{
-    int best = 0;
-    double cost = 0.0;
-    for (int kper = std::min(cap, kall); kper >= 1; --kper) {
-        const int nkr = (kall + kper - 1) / kper;
-        kper = (kall + nkr - 1) / nkr;  // the shortest march of as many ranges
-        const double t = (double)((base * nkr + slots - 1) / slots) * (kper + 1.5);
-        if (best == 0 || t < cost) {
-            cost = t;
-            best = kper;
-        }
-    }
-    return best;
-}
 
 // Hardware dispatch sends work-group b to XCD b % 8, and each XCD has its own
 // L2.  For a launch of n work-groups whose neighbours in logical order share

@@ -592,7 +592,7 @@ int launch_diffusion(nicam_ctx c, double *dscl, double *dscl_pl, const double *s
     // two work-groups per CU (registers).  us at levels per work-group: 18x18x42x40 21.8 at 3, 16.3 at 7 (one round),
     // 24.7 at 14; 34x34x78x40 81 at 13, 75 at 8; 66x66x98x40 289 at 49 (three rounds), 291 at 33, 318 at 10, 352 at 98;
     // 130x130x40x10 143 at 20, 132 at 14
-    A.kper = c->tune.diff_kper > 0 ? std::min(c->tune.diff_kper, D.kall) : level_split(base, D.kall, 512, D.kall);
+    A.kper = c->tune.diff_kper > 0 ? even_split(D.kall, c->tune.diff_kper) : level_split(base, D.kall, 512, D.kall);
     A.nkr = (D.kall + A.kper - 1) / A.kper;
     const long nmain = base * A.nkr;
     const long npole = dscl_pl ? (D.kall * kLallPl + CHUNK - 1) / CHUNK : 0;
@@ -661,7 +661,7 @@ int launch_divdamp(nicam_ctx c, double *const out[3], double *const out_pl[3], c
     // two work-groups per CU, one where the third slot's registers leave room for no more.  us at levels per
     // work-group: 18x18x42x40 32.8 at 3, 24.4 at 7 (one round), 33 at 14; 51x51x61x7 46.5 at 5, 36.5 at 10 (one round),
     // 51 at 20; 66x66x98x40 566 at 48 (three rounds), 600 at 32, 617 at 10, 687 at 96; 130x130x40x10 457 at 19, 430 at 13
-    A.kper = c->tune.ddmp_kper > 0 ? std::min(c->tune.ddmp_kper, nlev) : level_split(base, nlev, small ? 512 : 256, nlev);
+    A.kper = c->tune.ddmp_kper > 0 ? even_split(nlev, c->tune.ddmp_kper) : level_split(base, nlev, small ? 512 : 256, nlev);
     A.nkr = (nlev + A.kper - 1) / A.kper;
     const long nmain = base * A.nkr;
     const long npole = out_pl[0] ? (D.kall * kLallPl + CHUNK - 1) / CHUNK : 0;
