@@ -342,9 +342,14 @@ int launch_gradient(nicam_ctx c, double *grad, double *grad_pl, const double *sc
     A.have_pl = D.have_pl;
     A.nchunk = (D.gall + BLK - 1) / BLK;
     const long base = (long)A.nchunk * D.lall;
-    // four levels share a work-item's 21 coefficients, on every grid: 18x18x42x40 15.5 us at one level, 9.1 at 4;
-    // 34x34x42x10 10.8 at one, 7.4 at 4; 34x34x78x40 28.9 at 4, 30.9 at 10; 66x66x98x40 220 at one, 115 at 4, 126 at 20
-    A.kper = std::min(4, D.kall);
+    // Levels that share a work-item's 21 coefficients: as many as leave about 4096 work-groups, and at least four where
+    // those still fill the chip.  us, inputs from memory: 12x12x16 6.2 at one level, 7.4 at 4; 66x66x16 7.7 at one, 7.0
+    // at 2, 8.4 at 4; 34x34x60x2 9.2 at one, 8.6 at 4; 18x18x42x40 21.4 at one, 15.9 at 4; 34x34x78x40 52.4 at 4;
+    // 130x130x42x10 99 at 4, 92 at 6; 66x66x98x40 215 at 4, 186 at 17 (from the Infinity Cache 115 and 125);
+    // 130x130x42x40 363 at 4, 308 at 21; 514x514x42x4 563 at 4, 457 at 42
+    const long wg1 = base * D.kall;  // work-groups of one level each
+    const int nkr = (int)std::min((4096 + base - 1) / base, (long)D.kall);
+    A.kper = wg1 <= 256 ? 1 : wg1 <= 512 ? 2 : std::max(std::min(4, D.kall), (D.kall + nkr - 1) / nkr);
     A.nkr = (D.kall + A.kper - 1) / A.kper;
     const long nmain = base * A.nkr;
     const long npole = grad_pl ? (D.kall * kLallPl + BLK - 1) / BLK : 0;

@@ -236,10 +236,11 @@ def test_gpu_glue_kernels_match_oracle(gpu, oracle, gl, rl, kall):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("gl,rl,kall", [(7, 0, 11), (5, 1, 23), (3, 0, 4)])
+@pytest.mark.parametrize("gl,rl,kall", [(7, 0, 11), (5, 1, 23), (3, 0, 4), (3, 0, 41), (7, 0, 33)])
 def test_gpu_glue_kernels_match_oracle_over_level_ranges(gpu, oracle, gl, rl, kall):
     """Regions wide enough for a third staged cell per work-item, several level
-    ranges with a shorter last one, the fewest levels."""
+    ranges with a shorter last one, the fewest levels; the gradient at one, two,
+    four and five levels per work-group."""
     test_gpu_glue_kernels_match_oracle(gpu, oracle, gl, rl, kall)
 
 
