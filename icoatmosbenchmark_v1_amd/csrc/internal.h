@@ -73,7 +73,7 @@ struct Dims {
 struct nicam_tune {
     int hflux_kper = 0;   // levels per work-group in horizontal_flux
     int vlim_kchunk = 0;  // levels per work-item in vertical_limiter_thuburn
-    int vi_variant = 0;   // elimination-factor storage in vi_rhow_solver (1..4)
+    int vi_variant = 0;   // elimination-factor storage in vi_rhow_solver (1..5)
     int diff_kper = 0;    // levels per work-group in OPRT_diffusion
     int ddmp_kper = 0;    // levels per work-group in OPRT3D_divdamp
     int hlim_variant = 0; // horizontal limiter: 1 = streamed loads after the tile barrier, 2 = before it

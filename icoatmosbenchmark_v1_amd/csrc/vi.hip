@@ -4,7 +4,8 @@
 //
 // The reference builds the Helmholtz source Sall for a whole region, applies
 // the boundary conditions, then runs a Thomas elimination per column, all with
-// g innermost.  Here one work-item owns one column (g, l): the source term is
+// g innermost.  Here one work-item (or, in variant 5, one lane of each of four
+// waves) owns one column (g, l): the source term is
 // formed level by level inside the forward sweep (the level k-1 products are
 // carried in registers, so no Sall array exists), and a wavefront covers 64
 // consecutive g at one level, so all global traffic is contiguous.  The pole
@@ -423,15 +424,16 @@ __global__ void __launch_bounds__(BLOCK_CO) vi_kernel_coop(ViArgsT<Src> A)
 
 static_assert(BLOCK_CO == 256 && BLOCK_FAC == 256, "vi_group_kernel serves both");
 
-// several grids in one launch (cooperative, or a column per work-item): work-groups
-// [off[n], off[n+1]) belong to grid n
+// several grids in one launch: work-groups [off[n], off[n+1]) belong to grid n
 template <class Src>
 struct ViGroup {
     ViArgsT<Src> a[kMaxGroup];
     int off[kMaxGroup + 1];
     int n;
+    bool coop[kMaxGroup];  // cooperative, or a column per work-item
 };
 
+// COOP: some grid is cooperative
 template <class Src, bool COOP>
 __global__ void __launch_bounds__(256) vi_group_kernel(ViGroup<Src> G)
 {
@@ -440,16 +442,18 @@ __global__ void __launch_bounds__(256) vi_group_kernel(ViGroup<Src> G)
     while (n + 1 < G.n && b >= G.off[n + 1]) ++n;
     const ViArgsT<Src> &A = G.a[n];
     if constexpr (COOP) {
-        extern __shared__ double s_w[];
-        vi_coop_block<Src>(A, xcd_windowed(b - G.off[n], G.off[n + 1] - G.off[n], COWIN), s_w);
-    } else {
-        column_run<BLOCK_FAC>(A, b - G.off[n], [&](const ViFieldT<Src> &F, size_t base, size_t s) {
-            NoGamma gam;
-            int unused = 0;
-            vi_column<0, false, true>(F, base, s, A.kall, A.rdgzh, A.afact, A.bfact, A.dt, A.CVovRt2, A.alpha, A.grav,
-                                      gam, unused);
-        });
+        if (G.coop[n]) {
+            extern __shared__ double s_w[];
+            vi_coop_block<Src>(A, xcd_windowed(b - G.off[n], G.off[n + 1] - G.off[n], COWIN), s_w);
+            return;
+        }
     }
+    column_run<BLOCK_FAC>(A, b - G.off[n], [&](const ViFieldT<Src> &F, size_t base, size_t s) {
+        NoGamma gam;
+        int unused = 0;
+        vi_column<0, false, true>(F, base, s, A.kall, A.rdgzh, A.afact, A.bfact, A.dt, A.CVovRt2, A.alpha, A.grav,
+                                  gam, unused);
+    });
 }
 
 // The Thomas factorisation of one column (mod_vi.f90:218-231 without the
@@ -501,7 +505,20 @@ __global__ void __launch_bounds__(BLOCK_FAC) vi_factor_kernel(FactorArgs A)
 }
 
 constexpr int kMaxCoop = 320;  // levels whose column values fit 160 KiB of LDS
+constexpr int kTall = 160;     // above, one work-group of variant 5 fits a CU
 size_t coop_lds(int kall) { return sizeof(double) * 64 * kall; }
+
+// Whether variant 5 is faster than variant 2 on ncol columns of kall levels.  Measured, 5 over 2, FP64 and FP32 inputs:
+// few levels leave its waves nothing to share, which many columns do not forgive (40 x 66x66: 8 levels 1.74 and 1.71,
+// 16 1.11 and 1.15, 20 1.06 and 1.03, 26 0.95 and 0.94, 50 0.78 and 0.83; 10 x 34x34: 5 levels 1.29 and 1.34, 12 0.73
+// and 0.70), and above 160 levels a column per work-item hides its waits better once there are enough of them
+// (10 x 66x66 x 200 0.78 and 0.66; 20 x 0.92 and 0.93; 30 x 1.01 and 1.07; 40 x 0.92 and 1.12; 40 x 160 0.81 and 0.94).
+bool coop_wins(int kall, long ncol)
+{
+    if (kall > kMaxCoop) return false;
+    if (kall > kTall) return ncol <= 98304;
+    return kall >= 24 || ncol <= 8192L * (kall - 8);
+}
 
 template <class Src>
 void vi_make_args(nicam_ctx c, ViArgsT<Src> &A, double *w, double *w_pl, const Src *w0, const Src *w0_pl,
@@ -548,7 +565,7 @@ int launch_vi_t(nicam_ctx c, double *w, double *w_pl, const Src *w0, const Src *
     // inputs 332 against 400 (4); x 97 FP64 512 against 640 (2); 40 x 34x34 x 58 93 against 123 (2); 7 x 51x51 x 61
     // 57.6 against 98.7 (2); 12x12 x 98 31.3 against 32.6 (4).  At 42 levels the registers hold the column at two
     // waves per SIMD and 4 is as fast or faster (130x130 37.3 against 38.7, 10 x 66x66 68.1 against 71.9).
-    if (variant == 0) variant = D.kall == 42 ? 4 : (D.kall <= kMaxCoop ? 5 : 2);
+    if (variant == 0) variant = D.kall == 42 ? 4 : (coop_wins(D.kall, A.ncol) ? 5 : 2);
 
     if (variant == 1) {
         const size_t lds = sizeof(double) * BLOCK_LDS * D.kall;
@@ -625,22 +642,29 @@ int launch_vi_group_mixed(const nicam_ctx *cs, int n, const nicam_tracer_step_f3
     ViGroup<float> G;
     G.n = n;
     G.off[0] = 0;
-    int kmax = 0;
-    for (int i = 0; i < n; ++i) kmax = std::max(kmax, cs[i]->d.kall);
-    const bool coop = kmax <= kMaxCoop;
     for (int i = 0; i < n; ++i) {
         const nicam_ctx c = cs[i];
         const nicam_tracer_step_f32 &p = g[i];
         vi_make_args<float>(c, G.a[i], p.rhogw, p.rhogw_pl, p.rhogw0, p.rhogw0_pl, p.preg0, p.preg0_pl, p.rhog0,
                             p.rhog0_pl, p.Srho, p.Srho_pl, p.Sw, p.Sw_pl, p.Spre, p.Spre_pl, dt, c->RGAM32,
                             c->RGAM32_pl, c->RGAMH32, c->RGAMH32_pl, c->RGSGAM2_32, c->RGSGAM2_32_pl);
+    }
+    // The launch's LDS is the tallest cooperative grid's, for every grid: above 160 levels the others would run one
+    // work-group to a CU too, which they must be few for (one 34x34 region of 200 levels with 40 of 130x130 x 42 levels
+    // 726 us, 527 with its columns per work-item; of 300 levels with 40 of 66x66 x 60 271).
+    long all = 0;
+    int kmax = 0;
+    for (int i = 0; i < n; ++i) all += G.a[i].ncol;
+    for (int i = 0; i < n; ++i) {
         const ViArgsT<float> &a = G.a[i];
-        const long nb = coop ? column_blocks<64>(a.gall, a.lall, a.gall_pl, a.have_pl)
-                             : column_blocks<BLOCK_FAC>(a.gall, a.lall, a.gall_pl, a.have_pl);
+        G.coop[i] = coop_wins(a.kall, a.ncol) && (a.kall <= kTall || all <= 196608);
+        if (G.coop[i]) kmax = std::max(kmax, a.kall);
+        const long nb = G.coop[i] ? column_blocks<64>(a.gall, a.lall, a.gall_pl, a.have_pl)
+                                  : column_blocks<BLOCK_FAC>(a.gall, a.lall, a.gall_pl, a.have_pl);
         if ((long)G.off[i] + nb > 0x7fffffffL) return fail(NICAM_ERR_ARG, "group too large for one launch");
         G.off[i + 1] = G.off[i] + (int)nb;
     }
-    if (coop) {
+    if (kmax > 0) {
         const size_t lds = coop_lds(kmax);
         if (lds > 64 * 1024)
             NICAM_HIP(hipFuncSetAttribute((const void *)vi_group_kernel<float, true>,

@@ -357,7 +357,7 @@ def vi_variants(ctx, spec, steps, W) -> int:
     ctx.vi_rhow_getcoef(Mc, Mc_pl, Ml, Ml_pl, Mu, Mu_pl)
     for s in range(steps):
         ctx.vi_rhow_solver_putcoef(Mc, Mc_pl, Ml, Ml_pl, Mu, Mu_pl)
-        for v in (1, 2, 3, 4):
+        for v in (1, 2, 3, 4, 5):
             ctx.set_tuning(TUNE_VI_VARIANT, v)
             ctx.vi_rhow_solver(W["rhogw"], W["rhogw_pl"], *a64, 60.0)
             ctx.vi_rhow_solver_mixed(W["rhogw"], W["rhogw_pl"], *a32, 60.0)

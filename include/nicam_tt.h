@@ -88,8 +88,8 @@ int nicam_ctx_set_pointer_mode(nicam_ctx ctx, int mode);
  *                           0 = automatic.  The adjoint
  *                           follows it: 1 and 3 form the transposed
  *                           system's factors in the solve, 2, 4, 5 and 0
- *                           read the ones putcoef stores (0 at kall = 42: the
- *                           column in registers)
+ *                           read the ones putcoef stores (at kall = 42 only 2
+ *                           and 4 do: the others keep the column in registers)
  *   NICAM_TUNE_DIFF_KPER    levels per work-group of nicam_oprt_diffusion
  *   NICAM_TUNE_DDMP_KPER    levels per work-group of nicam_oprt3d_divdamp
  *   NICAM_TUNE_HLIM_VARIANT horizontal limiter, one tracer: 1 = the streamed
