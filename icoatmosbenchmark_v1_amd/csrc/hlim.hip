@@ -120,12 +120,16 @@ __device__ __forceinline__ void hlim_block(const HlimArgs<T> &A, int b)
         for (int tr = 0; tr < (MULTI ? A.ntr : 1); ++tr) hlim_pole(A, (b - A.nmain) * CHUNK + threadIdx.x, tr);
         return;
     }
-    // One tracer: work-groups in dispatch order, so that the eight XCDs sweep
-    // memory together (gl7 FP64 645 us, FP32 326, against 674 and 346 with an
-    // eighth of the launch to each XCD; the halo rows a chunk shares with the
-    // next are q, cmask and Qout_post of two rows, and the Infinity Cache
-    // serves them).  Many tracers: an eighth each (neutral at 8 tracers).
+    // One FP64 tracer: work-groups in dispatch order, so that the eight XCDs
+    // sweep memory together (66x66x98x40 637 us against 678 with an eighth of
+    // the launch to each XCD, 130x130x42x10 270 against 300; the halo rows a
+    // chunk shares with the next are q, cmask and Qout_post of two rows, and
+    // the Infinity Cache serves them).  FP32, whose chunks share more lines:
+    // windows of 32 work-groups an XCD (66x66x98x40 332 us, 328 in dispatch
+    // order, 344 in eighths; 258x258x42 45.7, 52.5 and 48.0; 34x34x78x40 55.3,
+    // 58.1 and 55.8).  Many tracers: an eighth each (neutral at 8 tracers).
     if (MULTI) b = (int)xcd_contiguous(b, A.nmain);
+    else if (sizeof(T) == 4) b = (int)xcd_windowed(b, A.nmain, 32);
     const int chunk = b % nchunk;
     const int kl = b / nchunk;
     const int k = kl % kall, l = kl / kall;

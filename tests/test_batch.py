@@ -46,7 +46,8 @@ def test_group_rejects_bad_sizes():
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("single", [False, True])
-@pytest.mark.parametrize("grid", [GRIDS[2], (258, 4, 1, 64, [1], True)], ids=["g34", "g258-wide-tiles"])
+@pytest.mark.parametrize("grid", [GRIDS[2], (258, 4, 1, 64, [1], True), (66, 16, 4, 68, [1, 0, 0, 1], True)],
+                         ids=["g34", "g258-wide-tiles", "g66-windows"])
 def test_gpu_batched_limiters_equal_single_tracer_calls(gpu, single, grid):
     import torch
 
