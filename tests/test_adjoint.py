@@ -490,18 +490,28 @@ def test_oracle_courant_derivative_fails_a_planted_slip(oracle):
 
 HLIM_GPU = [(6, 4, 2, 91, [1, 0]), (18, 6, 3, 92, [0, 1, 1]), (66, 12, 2, 93, [1, 0]), (130, 4, 1, 94, [0]),
             (160, 4, 1, 95, [1])]
+# pole rings of other sizes than six points (gall_pl), and more slabs than a work-group of the pole kernels
+RINGS = [(8, 40, 2, 96, [1, 0], 3), (8, 5, 2, 97, [0, 1], 5), (8, 4, 2, 98, [1, 0], 6), (8, 34, 2, 99, [1, 0], 15)]
+
+
+def _spec(c):
+    n, kall, lall, seed, sgp, *ring = c
+    return synth.GridSpec(n, kall, lall, gall_pl=ring[0] if ring else 6, have_pl=True, seed=seed), seed, sgp
+
+
+def _id(c):
+    return f"g{c[0]}k{c[1]}" + (f"-ring{c[5]}" if len(c) > 5 else "")
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("c", HLIM_GPU, ids=[f"g{c[0]}k{c[1]}" for c in HLIM_GPU])
+@pytest.mark.parametrize("c", HLIM_GPU + RINGS, ids=_id)
 def test_gpu_hlim_mask_and_adjoint_match_oracle(gpu, oracle, c):
     """Mask, q_a_b, q_b and Qout_post_b bit for bit (the GPU gathers every
     cotangent in the oracle's order), regions and poles; gall_1d up to 160,
     the widest region the kernels take."""
     import torch
 
-    n, kall, lall, seed, sgp = c
-    spec = synth.GridSpec(n, kall, lall, have_pl=True, seed=seed)
+    spec, seed, sgp = _spec(c)
     case = synth.make_case(spec, have_sgp=sgp)
     f = dict(case["hlim"])
     ctx = drivers.setup_context(spec, case["geo"])
@@ -544,15 +554,14 @@ def test_gpu_hlim_mask_and_adjoint_match_oracle(gpu, oracle, c):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("c", HLIM_GPU[:3], ids=[f"g{c[0]}k{c[1]}" for c in HLIM_GPU[:3]])
+@pytest.mark.parametrize("c", HLIM_GPU[:3] + RINGS, ids=_id)
 def test_gpu_hlim_adjoint_half_passes(gpu, oracle, c):
     """The faces alone (no Qout_prev_b) and the rows alone (no q_a_b, with
     ch_b) equal the oracle's adjoint with the other cotangent zero, bit for
     bit, and the faces-only pass writes no ch_b."""
     import torch
 
-    n, kall, lall, seed, sgp = c
-    spec = synth.GridSpec(n, kall, lall, have_pl=True, seed=seed)
+    spec, seed, sgp = _spec(c)
     case = synth.make_case(spec, have_sgp=sgp)
     f = dict(case["hlim"])
     ctx = drivers.setup_context(spec, case["geo"])
@@ -660,13 +669,12 @@ FLUX_GPU = [(6, 4, 2, 121, [1, 0]), (18, 4, 3, 122, [0, 1, 1]), (66, 5, 2, 123, 
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("c", FLUX_GPU, ids=[f"g{c[0]}k{c[1]}" for c in FLUX_GPU])
+@pytest.mark.parametrize("c", FLUX_GPU + RINGS, ids=_id)
 def test_gpu_flux_adjoint_matches_oracle(gpu, oracle, c):
     """Every cotangent bit for bit, the poles included."""
     import torch
 
-    n, kall, lall, seed, sgp = c
-    spec = synth.GridSpec(n, kall, lall, have_pl=True, seed=seed)
+    spec, seed, sgp = _spec(c)
     case = synth.make_case(spec, have_sgp=sgp)
     ctx = drivers.setup_context(spec, case["geo"])
     T = lambda a: torch.from_numpy(np.ascontiguousarray(a, np.float64)).to(gpu)  # noqa: E731
