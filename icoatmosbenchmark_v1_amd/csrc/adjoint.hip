@@ -5,6 +5,8 @@
 // reads, from the cotangent of its outputs.  Operation orders are fixed so
 // that the C restatement in the oracle gives the same bits.
 
+#include <type_traits>
+
 #include "internal.h"
 
 namespace nicam {
@@ -989,34 +991,53 @@ __global__ void __launch_bounds__(HSW) __attribute__((amdgpu_waves_per_eu(CHB ? 
 // is known at compile time (6, the ring every NICAM grid has): the ring's inputs
 // load at once and its sums stay in registers, where a walk through memory paid
 // a round trip per term (24 us at 98 levels, behind the regions' kernel; now
-// 10.5 us).  0: any size.
+// 10.5 us).  0: any size, through memory: indexed at run time, per-lane arrays
+// and selects over them take twice to three times as long (one 10x10 region and
+// the poles, 98 levels, rings of 5 and of 15 points: 22.9 us against 58.2 and
+// 42.6 against 140).
 template <int NPL>
 __global__ void __launch_bounds__(HPOLE) hlim_adjoint_pole(HaArgs A)
 {
     const int t = blockIdx.x * HPOLE + threadIdx.x;
     const int kall = A.kall, npl = NPL > 0 ? NPL : A.gall_pl;
-    constexpr int N = NPL > 0 ? NPL : kMaxGallPl, U = NPL > 0 ? NPL : 1;
+    constexpr int N = NPL > 0 ? NPL : 1, U = N;
     if (!A.have_pl || t >= kall * kLallPl) return;
     const int k = t % kall, l = t / kall;
     const size_t fb = ((size_t)l * kall + k) * npl;
     const size_t pplane = (size_t)kLallPl * kall * npl;
-    double qs[N], chs[N], cms[N];
-#pragma unroll U
-    for (int v = 0; v < N; ++v) {
-        const int u = v < npl ? v : 0;
-        qs[v] = A.q_pl[fb + u];
-        chs[v] = A.ch_pl[fb + u];
-        cms[v] = A.cmask_pl[fb + u];
+    // the ring's inputs, and the cotangents of q and of Qout_post's two bounds
+    std::conditional_t<(NPL > 0), double[N], const double *> qs, chs, cms;
+    std::conditional_t<(NPL > 0), double[N], double *> xq, xp0, xp1;
+    if constexpr (NPL > 0) {
+#pragma unroll
+        for (int v = 0; v < N; ++v) {
+            qs[v] = A.q_pl[fb + v];
+            chs[v] = A.ch_pl[fb + v];
+            cms[v] = A.cmask_pl[fb + v];
+            xq[v] = xp0[v] = xp1[v] = 0.0;
+        }
+    } else {
+        qs = A.q_pl + fb;
+        chs = A.ch_pl + fb;
+        cms = A.cmask_pl + fb;
+        xq = A.qb_pl + fb;
+        xp0 = A.Qpostb_pl ? A.Qpostb_pl + fb : nullptr;
+        xp1 = xp0 ? xp0 + pplane : nullptr;
+        for (int v = 0; v < npl; ++v) {
+            xq[v] = 0.0;
+            if (xp0) xp0[v] = xp1[v] = 0.0;
+        }
     }
     // the rows run when Qout_prev_b is given, the faces when q_a_b is
     double *xa = A.qab_pl ? A.qab_pl + fb : nullptr;
-    double xq[N], xp0[N], xp1[N];  // the cotangents of q and of Qout_post's two bounds
-#pragma unroll U
-    for (int v = 0; v < N; ++v) xq[v] = xp0[v] = xp1[v] = 0.0;
     // x[i] += y where the index is known at run time only
-    auto add = [&](double (&x)[N], int i, double y) {
-#pragma unroll U
-        for (int v = 0; v < N; ++v) x[v] = v == i ? x[v] + y : x[v];
+    auto add = [&](auto &x, int i, double y) {
+        if constexpr (NPL > 0) {
+#pragma unroll
+            for (int v = 0; v < N; ++v) x[v] = v == i ? x[v] + y : x[v];
+        } else {
+            x[i] = x[i] + y;
+        }
     };
     const double BIG = A.big;
     auto arc = [&](int v, int &il, int &ih, double &lo_v, double &hi_v) {
@@ -1096,8 +1117,7 @@ __global__ void __launch_bounds__(HPOLE) hlim_adjoint_pole(HaArgs A)
         xq[0] = xq[0] + (fac + zerosw) * bq;
         int selc = 0;
         double selm = 1.0;
-#pragma unroll U
-        for (int v = 1; v < npl; ++v) {
+        auto pick = [&](int v) {
             int il, ih;
             double lv, hv;
             arc(v, il, ih, lv, hv);
@@ -1105,6 +1125,12 @@ __global__ void __launch_bounds__(HPOLE) hlim_adjoint_pole(HaArgs A)
                 selc = mm == 0 ? ih : il;
                 selm = cms[v];
             }
+        };
+        if constexpr (NPL > 0) {
+#pragma unroll
+            for (int v = 1; v < npl; ++v) pick(v);
+        } else if (sel >= 0) {
+            pick(sel);
         }
         add(xq, selc, (-(fac * E) * selm) * bq);
 #pragma unroll U
@@ -1138,12 +1164,14 @@ __global__ void __launch_bounds__(HPOLE) hlim_adjoint_pole(HaArgs A)
         else if (kind == 2) add(xp1, T, ob);
         else if (kind >= 3) add(xq, cell, ob);
     }
-#pragma unroll U
-    for (int v = 0; v < npl; ++v) {
-        A.qb_pl[fb + v] = xq[v];
-        if (A.Qpostb_pl) {
-            A.Qpostb_pl[fb + v] = xp0[v];
-            A.Qpostb_pl[pplane + fb + v] = xp1[v];
+    if constexpr (NPL > 0) {
+#pragma unroll
+        for (int v = 0; v < npl; ++v) {
+            A.qb_pl[fb + v] = xq[v];
+            if (A.Qpostb_pl) {
+                A.Qpostb_pl[fb + v] = xp0[v];
+                A.Qpostb_pl[pplane + fb + v] = xp1[v];
+            }
         }
     }
 }
