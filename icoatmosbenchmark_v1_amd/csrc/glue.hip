@@ -163,10 +163,10 @@ __device__ void remap_pole(const RemapArgs &A, long p)
 // its six faces by that face's own mask: faces 1-3 from its own arcs, faces
 // 4-6 from the arcs of im1j (AI), im1jm1 (AIJ) and ijm1 (AJ).  A face no arc
 // reaches keeps its value.  The next level's inputs are loaded into registers
-// while phase 2 stores this one's faces (34x34x78x40 198 us with the loads
-// waited for at the head of each level and three barriers, 166 now; 66x66x98x40
-// 872 -> 753).  NSTG: staged cells per
-// work-item, NSTG * RCH >= RCH + 2 * gall_1d + 2.
+// while phase 2 stores this one's faces (34x34x78x40 196 us with the loads
+// waited for at the head of each level and three barriers, 181 now; 66x66x98x40
+// 870 -> 801).  NSTG: staged cells per work-item,
+// NSTG * RCH >= RCH + 2 * gall_1d + 2.
 template <int NSTG>
 __global__ void __launch_bounds__(RCH) remap_kernel(RemapArgs A)
 {

@@ -366,14 +366,18 @@ int hflux_launch(void (*const k[4])(Arg), int v, long nblk, size_t lds, hipStrea
 // Levels per work-group for base chunks of kall levels each.  The chip runs
 // SLOTS work-groups at a time (two per CU in FP64, by registers; four in FP32),
 // and each pays about one and a half levels for its metrics, so a launch costs
-// rounds * (levels + 1.5): the least of that over all splits, the longer march
-// on a tie.  FP64, us at kper: one 130x130x42 region 46.6 at 1, 39 at 2, 36 at 3,
-// 39 at 4, 35 at 6 (one round), 39.6 at 8, 49 at 14; 40 regions of 18x18x42 43 at
-// 1, 36 at 4, 32 at 7 (one round), 43 at 14; 34x34x78 155 at 4, 144 at 8, 152 at
-// 13, 178 at 26; 66x66x98 596 at 25 and 49, 617 at 33, 713 at 98: the order the
-// cost gives, every time.  FP32 keeps more work-groups in flight and gains from
-// short marches at any size (66x66x98 399 at 98, 359 at 33, 332 at 10; 130x130x98
-// 1238 at 49, 1195 at 14), hence its cap.
+// about rounds * (levels + 1.5).  FP64, us at kper: one 130x130x42 region 46.6 at
+// 1, 39 at 2, 36 at 3, 39 at 4, 35 at 6 (one round), 39.6 at 8, 49 at 14; 40
+// regions of 18x18x42 43 at 1, 36 at 4, 32 at 7 (one round), 43 at 14; 34x34x78
+// 155 at 4, 144 at 8, 152 at 13, 178 at 26; 66x66x98 596 at 25 and 49, 617 at 33,
+// 713 at 98.  The least of it is not always the fastest, but near: of 25 lengths
+// tried at each of 42 sizes from 12x12x16 to 514x514x42, both precisions, the one
+// taken is within 3.3 % of the best but at two (7 % at 7 x 51x51x61 FP64, 38 us
+// against 35.5 at 5; 4.5 % at 514x514x42 FP32).  The widest instances, whose tiles
+// leave one work-group to a CU, are among the others.
+// In FP32 the cost favours few long marches that fit one round, the time does not
+// (66x66x98: 398 at 98, which it would take, 359 at 33, 328 at 14, 326 at 15;
+// 130x130x98 1238 at 49, 1195 at 14; but 130x130x42 532 at 14, 526 at 28): the cap.
 template <class T>
 int hflux_kper(long base, int kall)
 {

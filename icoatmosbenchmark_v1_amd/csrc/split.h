@@ -16,8 +16,8 @@ inline int even_split(int kall, int kper)
 // Levels per work-group, at most cap, of a kernel whose work-groups march up a
 // range of levels: base columns of work-groups over kall levels, slots of them
 // on the chip at a time, each paying about one and a half levels to start.  The
-// launch costs rounds * (levels + 1.5); the least of that, the longer march on
-// a tie.
+// launch costs about rounds * (levels + 1.5): the least of that, the longer march
+// on a tie.  An estimate: the kernels say how near it comes.
 inline int level_split(long base, int kall, long slots, int cap)
 {
     int best = 0;

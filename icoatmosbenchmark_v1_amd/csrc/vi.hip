@@ -279,8 +279,9 @@ constexpr int NW = 4, BLOCK_CO = 64 * NW;
 constexpr int CB = 4;   // levels of source loads in flight per wave
 constexpr int CD = 16;  // levels of factors in flight in the recurrences
 // 64 columns of a level row end inside cache lines that the next 64 share: COWIN
-// consecutive work-groups run on one XCD (gl7 step 1802 -> 1745 us; 4: 1787, an
-// eighth of the launch to each XCD: 1816)
+// consecutive work-groups run on one XCD (66x66x98x40, us: FP64 350 at 16, 352
+// at 4, 354 in dispatch order, 362 with an eighth of the launch to each XCD; FP32
+// inputs 252, 254, 263 and 263)
 constexpr int COWIN = 16;
 constexpr int CG = 16;  // levels of the final scaling in flight per wave
 
@@ -561,10 +562,10 @@ int launch_vi_t(nicam_ctx c, double *w, double *w_pl, const Src *w0, const Src *
     int variant = c->tune.vi_variant;
     const bool reg_ok = (D.kall == 42 || D.kall == 98);
     if (((variant == 3 || variant == 4) && !reg_ok) || (variant == 5 && D.kall > kMaxCoop)) variant = 0;
-    // measured with the v-limiter (us; 5 against the best other): 40 x 66x66 x 98 FP64 506 against 533 (4), FP32
-    // inputs 332 against 400 (4); x 97 FP64 512 against 640 (2); 40 x 34x34 x 58 93 against 123 (2); 7 x 51x51 x 61
-    // 57.6 against 98.7 (2); 12x12 x 98 31.3 against 32.6 (4).  At 42 levels the registers hold the column at two
-    // waves per SIMD and 4 is as fast or faster (130x130 37.3 against 38.7, 10 x 66x66 68.1 against 71.9).
+    // us, 5 against the best other: 40 x 66x66 x 98 FP64 354 and 371 (4), FP32 inputs 253 and 321 (4); 40 x 34x34 x 58
+    // 53 and 85 (2), 36 and 63; 7 x 51x51 x 61 32 and 58 (2), 26 and 63; 12x12 x 98 26.7 and 29.1 (4).  At 42 levels the
+    // registers hold the column at two waves per SIMD: inputs from the caches, 4 takes 12.0 on one 34x34 region, 160 on
+    // 40 x 66x66, 594 on 40 x 130x130, 5 15.1, 157 and 607; from memory 28.7, 218 and 656 against 22.8, 210 and 657.
     if (variant == 0) variant = D.kall == 42 ? 4 : (coop_wins(D.kall, A.ncol) ? 5 : 2);
 
     if (variant == 1) {

@@ -10,7 +10,7 @@
             mixed rho*w solve, the conservative and vertical updates, the
             mass sums; the limiter with the library's own Qout exchange
             (FP64 and FP32) and one COMM_data_transfer
-  vi        every rho*w solve variant (1-4) with FP64 and FP32 inputs, the
+  vi        every rho*w solve variant (1-5) with FP64 and FP32 inputs, the
             factorisation (putcoef) and both adjoint variants
   batched   the grouped multi-tracer step on the gl5-gl8 grids (32 tracers)
   extras    OPRT_diffusion, OPRT3D_divdamp, the horizontal and vertical step
